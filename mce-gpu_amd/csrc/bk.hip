@@ -2226,15 +2226,24 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
   s.cover = pr.cover + (uint64_t)gw * kWave;
   const uint32_t *items1 = (const uint32_t *)pr.items;
   const uint2 *items2 = (const uint2 *)pr.items;
-  // phase 1: first-level subproblems by ticket
+  // phase 1: first-level subproblems by ticket. A wave's first ticket is its
+  // position in the grid (neighbouring tickets, the heaviest, on different
+  // workgroups, so that they do not share a CU's LDS pool), the next ones
+  // come from the counter: 11 ns each on its line, 45 us a launch of 4096
+  // waves when their first ones came from it too.
+  const uint32_t nwaves = gridDim.x * pr.wpg;
+  uint32_t tickets = 0;
   while (true) {
     clk.to(kBdQueue);
-    uint32_t t = 0;
-    if (L == 0) {
-      t = atomicAdd(pr.ticket, 1u);
-      if (pr.host_progress && (t & 1023u) == 0) post_progress(pr.host_progress, t);
+    uint32_t t = wig * gridDim.x + blockIdx.x;
+    if (tickets) {
+      if (pr.n_items <= pr.t1 && pr.n_items <= nwaves) break;  // one each and no more
+      if (L == 0) {
+        t = nwaves + atomicAdd(pr.ticket, 1u);
+        if (pr.host_progress && (t & 1023u) == 0) post_progress(pr.host_progress, t);
+      }
+      t = uniform(t);
     }
-    t = uniform(t);
     uint64_t lo, hi;
     if (t < pr.t1) {
       lo = t;
@@ -2245,6 +2254,7 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
     }
     if (lo >= pr.n_items) break;
     hi = min(hi, pr.n_items);
+    ++tickets;
     clk.to(kBdInduced);
     for (uint64_t it = lo; it < hi; ++it) {
       wa.sub_cliques = 0;
@@ -2360,8 +2370,10 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
         pool_put(pl, rg);
       }
     }
-    if (kWL && L == 0) atomicSub(pr.ctl + kCtlOutstanding, 1ull);
   }
+  // (the launch cannot end before this wave gets here: its tickets leave the
+  // outstanding count together)
+  if (kWL && L == 0 && tickets) atomicSub(pr.ctl + kCtlOutstanding, (unsigned long long)tickets);
   // phase 2: donated subtrees until no work is outstanding. An idle wave puts
   // itself on the idle queue and waits on its own mailbox line; a donor takes
   // it off the queue and writes the task into its slot, so no line is polled
@@ -2524,11 +2536,6 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
   }
   clk.to(kBdOther);
   if (L == 0) {
-    atomicAdd(&pr.acc[kAccCount], (unsigned long long)wa.count);
-    atomicAdd(&pr.acc[kAccHash], (unsigned long long)wa.hash);
-    atomicAdd(&pr.acc[kAccNodes], (unsigned long long)wa.nodes);
-    atomicAdd(&pr.acc[kAccDonations], (unsigned long long)wa.donations);
-    atomicMax(&pr.acc[kAccMaxSize], (unsigned long long)wa.max_size);
     if (pr.wave_val) {
       pr.wave_val[gw] = kStat == kStatDonor ? wa.donations : wa.nodes;
       pr.wave_cu[gw] = hw_cu_id();
@@ -2538,7 +2545,25 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
         for (int i = 0; i < 7; ++i) pr.wave_bd[(uint64_t)gw * 7 + i] = clk.acc[i];
     }
   }
+  // totals: summed over the workgroup in the pool's mask words (the pool is
+  // done), one update each and workgroup (five by every wave, on one line,
+  // were 0.2 ms of every launch)
+  unsigned long long *tot = (unsigned long long *)pl.mask;
+  static_assert(kPoolWords >= 5 && kAccCount == 0 && kAccHash == 1 && kAccNodes == 2 && kAccDonations == 3,
+                "tot[0..3] in the order of acc, then the maximum size");
   __syncthreads();
+  if (threadIdx.x < 5) tot[threadIdx.x] = 0;
+  __syncthreads();
+  if (L == 0 && wa.nodes + wa.count) {
+    atomicAdd(&tot[kAccCount], (unsigned long long)wa.count);
+    atomicAdd(&tot[kAccHash], (unsigned long long)wa.hash);
+    atomicAdd(&tot[kAccNodes], (unsigned long long)wa.nodes);
+    atomicAdd(&tot[kAccDonations], (unsigned long long)wa.donations);
+    atomicMax(&tot[4], (unsigned long long)wa.max_size);
+  }
+  __syncthreads();
+  if (threadIdx.x < 4 && tot[threadIdx.x]) atomicAdd(&pr.acc[threadIdx.x], tot[threadIdx.x]);
+  if (threadIdx.x == 4 && tot[4] > ld_relaxed(&pr.acc[kAccMaxSize])) atomicMax(&pr.acc[kAccMaxSize], tot[4]);
   for (uint32_t i = threadIdx.x; i < pr.hist_lds; i += blockDim.x)
     if (hist_lds[i]) atomicAdd(&pr.hist[min(i, pr.hist_len - 1)], hist_lds[i]);
 }
@@ -2584,8 +2609,17 @@ __global__ void need_kernel(const uint64_t *rp, const uint64_t *split, const voi
     mx = max(mx, (unsigned long long)need);
     over += need > cap;
   }
-  atomicMax(&out[0], mx);
-  if (over) atomicAdd(&out[1], over);
+  // one update per workgroup, and only of a maximum that it raises
+  __shared__ unsigned long long smx, sover;
+  if (threadIdx.x == 0) smx = sover = 0;
+  __syncthreads();
+  atomicMax(&smx, mx);
+  if (over) atomicAdd(&sover, over);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    if (smx > ld_relaxed(&out[0])) atomicMax(&out[0], smx);
+    if (sover) atomicAdd(&out[1], sover);
+  }
 }
 
 template <bool kIPX, bool kWL, int kStat>
@@ -2732,8 +2766,8 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
                      MCE_MAX_OUT_DEGREE);
   int dev = 0;
   MCE_HIP(hipGetDevice(&dev));
-  hipDeviceProp_t prop;
-  MCE_HIP(hipGetDeviceProperties(&prop, dev));
+  int cus = 0;
+  MCE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   // the lane solver runs in its own kernel instance (IPX, no statistics)
   const uint32_t ls_max = stat_of(cfg.task) == kStatNone && cfg.ipx ? std::min<uint32_t>(cfg.lane_max, kLsMax) : 0;
   const int stat = ls_max ? kStatLane : stat_of(cfg.task);
@@ -2804,7 +2838,7 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
   // hub row filter: 64 words per wave, for every wave a launch can hold (four
   // per SIMD), taken before the arenas size themselves to what is left
   uint64_t *cover = nullptr;
-  const uint32_t max_waves = (uint32_t)prop.multiProcessorCount * 16;
+  const uint32_t max_waves = (uint32_t)cus * 16;
   if (cfg.ipx && (rc = dmalloc((void **)&cover, 8ull * kWave * max_waves, kWsCover))) return rc;
   // per-wave HBM arena cap: items that need more are deferred to a second
   // pass with arenas sized for the largest. From a scratch region, one
@@ -2812,7 +2846,7 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
   // pass.
   uint64_t cap = cfg.hbm_bytes ? cfg.hbm_bytes : 16ull << 20;
   if (sc) cap = std::min<uint64_t>(cap, (sc->left() / wpg) & ~255ull);
-  need_kernel<<<1024, 256, 0, s>>>(g.rp, g.split, d_items, n_items, (uint32_t)cfg.level, cfg.ipx, cap, need);
+  need_kernel<<<(uint32_t)std::min<uint64_t>(1024, (n_items + 255) / 256), 256, 0, s>>>(g.rp, g.split, d_items, n_items, (uint32_t)cfg.level, cfg.ipx, cap, need);
   unsigned long long hneed[2];
   MCE_HIP(hipMemcpyAsync(hneed, need, sizeof(hneed), hipMemcpyDeviceToHost, s));
   MCE_HIP(hipStreamSynchronize(s));
@@ -2825,7 +2859,7 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
   if ((rc = dispatch(cfg.ipx, cfg.wl, stat, true, &nb, pr, 0, wpg, lds, s))) return rc;
   nb = std::max(nb, 1);
   if (cfg.groups_per_cu) nb = std::min<int>(nb, (int)cfg.groups_per_cu);
-  uint32_t groups = (uint32_t)(nb * prop.multiProcessorCount);  // all waves co-resident
+  uint32_t groups = (uint32_t)(nb * cus);  // all waves co-resident
   uint64_t arena = std::min<uint64_t>(hneed[0], cap);
   arena = (arena + 255) & ~255ull;
   size_t freeb = 0, totalb = 0;
@@ -2861,6 +2895,8 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
     const uint64_t per_slot = budget / ((uint64_t)groups * wpg);
     slot_xcap = std::min<uint64_t>(want_x, (per_slot - slot_fixed - 512) / slot_per_x);
   }
+  // without the worker list, workgroups past one per item have nothing to do
+  if (!cfg.wl && !wave_stats) groups = (uint32_t)std::min<uint64_t>(groups, n_items);
   const uint32_t waves = groups * wpg;
 
   uint8_t *hbm = nullptr;
@@ -2913,7 +2949,8 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
   pr.wave_bd = wave_bd;
   pr.wpg = wpg;
   const uint64_t n_tickets = n_items <= pr.t1 ? n_items : pr.t1 + (n_items - pr.t1 + pr.chunk - 1) / pr.chunk;
-  if (n_tickets >= 0xFFFFFF00ull) return set_error(MCE_ELIMIT, "too many work tickets");
+  // (a wave's claims run past the last ticket by at most one, from `waves` on)
+  if (n_tickets + 2ull * waves >= 0xFFFFFF00ull) return set_error(MCE_ELIMIT, "too many work tickets");
   if (cfg.wl) {
     pr.slot_pmax = slot_pmax;
     pr.slot_wmax = slot_wmax;

@@ -324,7 +324,7 @@ __global__ __launch_bounds__(256) void predict_kernel(uint64_t rows, const float
 
 // Schedule keys from predictions: key = clamp(64 * pred, 0, 4095); counts
 // non-finite predictions; accumulates the predicted work sum and maximum.
-__global__ void keys_kernel(uint32_t n, const float *__restrict__ pred, uint32_t *__restrict__ key,
+__global__ __launch_bounds__(256) void keys_kernel(uint32_t n, const float *__restrict__ pred, uint32_t *__restrict__ key,
                             unsigned int *bad, float *work) {
   float s = 0.f, mx = 0.f;
   uint32_t nb = 0;
@@ -341,8 +341,21 @@ __global__ void keys_kernel(uint32_t n, const float *__restrict__ pred, uint32_t
     mx = fmaxf(mx, w);
   }
   if (nb) atomicAdd(bad, nb);
-  atomicAdd(&work[0], s);
-  atomicMax((unsigned int *)&work[1], __float_as_uint(mx));  // non-negative floats order as their bits
+  // one update per workgroup (an update by every thread took 0.1 ms)
+  __shared__ float ssum[4];
+  __shared__ unsigned int smax;
+  if (threadIdx.x == 0) smax = 0;
+  __syncthreads();
+  s = wave_sum_f32(s);
+  atomicMax(&smax, __float_as_uint(mx));  // non-negative floats order as their bits
+  if (lane_id() == 0) ssum[threadIdx.x / kWave] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (uint32_t w = 1; w < blockDim.x / kWave; ++w) s += ssum[w];
+    if (s != 0.f) atomicAdd(&work[0], s);
+    if (smax > __hip_atomic_load((unsigned int *)&work[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax((unsigned int *)&work[1], smax);
+  }
 }
 
 struct DevBuf {
@@ -435,7 +448,7 @@ int learned_keys(const DevGraph &g, const OrderInfo &info, const mce_mlp &m, uin
   if ((rc = predict_device(m, F, g.n, pred, s))) return rc;
   MCE_HIP(hipMemsetAsync(work, 0, 2 * sizeof(float), s));
   MCE_HIP(hipMemsetAsync(bad, 0, sizeof(unsigned int), s));
-  keys_kernel<<<1024, 256, 0, s>>>(g.n, pred, keys, bad, work);
+  keys_kernel<<<(uint32_t)std::min<uint64_t>(1024, (g.n + 255ull) / 256), 256, 0, s>>>(g.n, pred, keys, bad, work);
   float hw[2];
   unsigned int hb = 0;
   MCE_HIP(hipMemcpyAsync(hw, work, sizeof(hw), hipMemcpyDeviceToHost, s));
