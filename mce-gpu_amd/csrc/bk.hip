@@ -29,8 +29,9 @@
 // subtree expands exactly as it would have in the donor.
 //
 // Worker list: an idle wave puts its id on a bounded lock-free queue in HBM
-// (per-slot sequence numbers, agent-scope acquire/release so that a slot
-// written on one XCD is seen on another) and waits on its own mailbox line.
+// (per-slot sequence numbers; what one wave hands another, on any XCD, goes
+// through agent-scope stores and loads, never through fences) and waits on
+// its own mailbox line.
 // A busy wave whose task has run long enough takes an idle wave off the queue
 // and writes into that wave's task slot the next candidate of its shallowest
 // frame (the largest remaining subtree): its P and X words, the donor's vertex
@@ -236,27 +237,62 @@ __device__ __forceinline__ uint64_t full_word(uint32_t p) {
   return (L == W - 1 && (p & 63)) ? ((1ull << (p & 63)) - 1) : ~0ull;
 }
 
+// Words handed from one wave to another, on any XCD: agent-scope stores and
+// loads, which go past the caches that are not shared, so that no fence is
+// needed around them. An agent-scope release writes the whole L2 of the XCD
+// back and an acquire empties the caches under the waves still at work: with
+// them a hand-over cost 1.7 us of the whole launch (R-MAT 13, IP, donating at
+// 10 us: 69,000 donations in 130 ms). Without them, default settings: R-MAT 13
+// IP 13.3 -> 6.9 ms, Chung-Lu 30,011 11.1 -> 4.1, R-MAT 14 40.8 -> 29.6,
+// Chung-Lu 2^18 121 -> 111.
+template <class T>
+__device__ __forceinline__ void st_shared(T *p, T v) {
+  __hip_atomic_store((__attribute__((address_space(1))) T *)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ T ld_shared(const T *p) {
+  return __hip_atomic_load((__attribute__((address_space(1))) T *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// This wave's earlier stores have reached their scope and its loads have
+// returned; the compiler moves no access across.
+__device__ __forceinline__ void drain() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_s_waitcnt(0);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Forward wave copies, four loads in flight per lane; each chunk of 256
 // elements is read before it is written, so a destination below an
-// overlapping source is safe.
-template <class T>
+// overlapping source is safe. kOut / kIn: the destination / source is a task
+// slot (st_shared, ld_shared).
+template <class T, bool kOut, bool kIn>
 __device__ __forceinline__ void wave_copy_t(T *dst, const T *src, uint64_t n) {
   const uint32_t L = lane_id();
+  auto get = [&](uint64_t i) -> T {
+    if constexpr (kIn) return i < n ? ld_shared(src + i) : T(0);
+    else return i < n ? src[i] : T(0);
+  };
+  auto put = [&](uint64_t i, T x) {
+    if (i >= n) return;
+    if constexpr (kOut) st_shared(dst + i, x);
+    else dst[i] = x;
+  };
   for (uint64_t b = 0; b < n; b += 4 * kWave) {
     const uint64_t i0 = b + L, i1 = i0 + kWave, i2 = i1 + kWave, i3 = i2 + kWave;
-    const T x0 = i0 < n ? src[i0] : T(0), x1 = i1 < n ? src[i1] : T(0);
-    const T x2 = i2 < n ? src[i2] : T(0), x3 = i3 < n ? src[i3] : T(0);
-    if (i0 < n) dst[i0] = x0;
-    if (i1 < n) dst[i1] = x1;
-    if (i2 < n) dst[i2] = x2;
-    if (i3 < n) dst[i3] = x3;
+    const T x0 = get(i0), x1 = get(i1), x2 = get(i2), x3 = get(i3);
+    put(i0, x0);
+    put(i1, x1);
+    put(i2, x2);
+    put(i3, x3);
   }
 }
+template <bool kOut = false, bool kIn = false>
 __device__ __forceinline__ void wave_copy(uint32_t *dst, const uint32_t *src, uint32_t n) {
-  wave_copy_t<uint32_t>(dst, src, n);
+  wave_copy_t<uint32_t, kOut, kIn>(dst, src, n);
 }
+template <bool kOut = false, bool kIn = false>
 __device__ __forceinline__ void copy64(uint64_t *dst, const uint64_t *src, uint64_t n) {
-  wave_copy_t<uint64_t>(dst, src, n);
+  wave_copy_t<uint64_t, kOut, kIn>(dst, src, n);
 }
 
 // Typed arena accesses: kL picks LDS (ds_*) over global memory (global_*).
@@ -643,8 +679,7 @@ __device__ __forceinline__ unsigned long long ring_claim_push(const BkParams &pr
   unsigned long long *seq = pr.seq + (uint64_t)q * pr.ring_cap;
   unsigned long long pos = ld_relaxed(tail);
   for (int it = 0; it < 8; ++it) {
-    const unsigned long long sq =
-        __hip_atomic_load(&seq[pos % pr.ring_cap], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long sq = ld_relaxed(&seq[pos % pr.ring_cap]);
     const long long dif = (long long)(sq - pos);
     if (dif == 0) {
       if (__hip_atomic_compare_exchange_weak(tail, &pos, pos + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
@@ -666,8 +701,7 @@ __device__ __forceinline__ unsigned long long ring_claim_pop(const BkParams &pr,
   unsigned long long *seq = pr.seq + (uint64_t)q * pr.ring_cap;
   unsigned long long pos = ld_relaxed(head);
   for (int it = 0; it < 8; ++it) {
-    const unsigned long long sq =
-        __hip_atomic_load(&seq[pos % pr.ring_cap], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long sq = ld_relaxed(&seq[pos % pr.ring_cap]);
     const long long dif = (long long)(sq - (pos + 1));
     if (dif == 0) {
       if (__hip_atomic_compare_exchange_weak(head, &pos, pos + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
@@ -723,8 +757,9 @@ __device__ __forceinline__ uint32_t claim_receiver(const BkParams &pr, uint32_t 
       const unsigned long long pos = ring_claim_pop(pr, q);
       if (pos != kNoSlot) {
         const uint64_t at = (uint64_t)q * pr.ring_cap + pos % pr.ring_cap;
-        r = __hip_atomic_load(&pr.idle_ids[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&pr.seq[at], pos + pr.ring_cap, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        r = ld_shared(&pr.idle_ids[at]);
+        drain();  // the id is read before its queue entry is free again
+        st_shared(&pr.seq[at], pos + pr.ring_cap);
         atomicAdd(pr.ctl + kCtlOutstanding, 1ull);
       }
     }
@@ -732,11 +767,23 @@ __device__ __forceinline__ uint32_t claim_receiver(const BkParams &pr, uint32_t 
   return uniform(r);
 }
 
+// A task's header, written by lane 0 as 64-bit words: {root, |R|}, {|S|, W},
+// {outside rows or ids, kind}, R's hash sum.
+__device__ __forceinline__ void put_header(uint8_t *slot, uint32_t root, uint32_t rsize, uint32_t p, uint32_t W,
+                                           uint32_t nx, uint32_t kind, uint64_t mix) {
+  if (lane_id() == 0) {
+    uint64_t *h = (uint64_t *)slot;
+    st_shared(h, (uint64_t)rsize << 32 | root);
+    st_shared(h + 1, (uint64_t)W << 32 | p);
+    st_shared(h + 2, (uint64_t)kind << 32 | nx);
+    st_shared(h + 3, mix);
+  }
+}
+
 // Hands the task written into receiver r's slot over to it.
 __device__ __forceinline__ void publish_task(const BkParams &pr, uint32_t r) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-  if (lane_id() == 0)
-    __hip_atomic_store(&pr.mbox[(uint64_t)r * kMboxStride], 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+  drain();  // the slot is written
+  if (lane_id() == 0) st_shared(&pr.mbox[(uint64_t)r * kMboxStride], 1ull);
 }
 
 // Puts this idle wave on its XCD's idle queue (its mailbox cleared first);
@@ -744,12 +791,13 @@ __device__ __forceinline__ void publish_task(const BkParams &pr, uint32_t r) {
 __device__ __forceinline__ bool register_idle(const BkParams &pr, uint32_t gw, uint32_t xq) {
   unsigned long long pos = kNoSlot;
   if (lane_id() == 0) {
-    __hip_atomic_store(&pr.mbox[(uint64_t)gw * kMboxStride], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    st_shared(&pr.mbox[(uint64_t)gw * kMboxStride], 0ull);
     pos = ring_claim_push(pr, xq);
     if (pos != kNoSlot) {
       const uint64_t at = (uint64_t)xq * pr.ring_cap + pos % pr.ring_cap;
-      __hip_atomic_store(&pr.idle_ids[at], gw, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(&pr.seq[at], pos + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+      st_shared(&pr.idle_ids[at], gw);
+      drain();  // mailbox and id are written before the entry is published
+      st_shared(&pr.seq[at], pos + 1);
     }
   }
   return uniform64(pos) != kNoSlot;
@@ -807,26 +855,14 @@ __device__ __forceinline__ bool donate_shallowest(const BkParams &pr, Sub &s, ui
     const uint32_t rcv = claim_receiver(pr, wa.xq);
     if (rcv == kNone) return false;
     uint8_t *slot = pr.ring + (uint64_t)rcv * pr.slot_bytes;
-    if (L == 0) {
-      uint32_t *h = (uint32_t *)slot;
-      h[0] = s.root;
-      h[1] = s.rsize + j + 1;
-      h[2] = s.p;
-      h[3] = W;
-      h[4] = nx;
-      h[5] = kTaskList;
-      *(uint64_t *)(slot + 24) = mixj + splitmix64(s.S[c]);
-    }
+    put_header(slot, s.root, s.rsize + j + 1, s.p, W, nx, kTaskList, mixj + splitmix64(s.S[c]));
     uint64_t *sp = (uint64_t *)(slot + pr.slot_oP);
     if (act) {
-      sp[L] = Pn;
-      sp[pr.slot_wmax + L] = Xn;
+      st_shared(sp + L, Pn);
+      st_shared(sp + pr.slot_wmax + L, Xn);
     }
-    uint32_t *sS = (uint32_t *)(slot + pr.slot_oS);
-    for (uint32_t i = L; i < s.p; i += kWave) sS[i] = s.S[i];
-    uint64_t *sA = (uint64_t *)(slot + pr.slot_oA);
-    const uint64_t nA = (uint64_t)s.p * W;
-    copy64(sA, s.A, nA);
+    wave_copy<true>((uint32_t *)(slot + pr.slot_oS), s.S, s.p);
+    copy64<true>((uint64_t *)(slot + pr.slot_oA), s.A, (uint64_t)s.p * W);
     uint32_t *sXI = (uint32_t *)(slot + pr.slot_oXI);
     uint64_t *sXR = (uint64_t *)(slot + pr.slot_oXR);
     uint32_t w = 0;
@@ -842,10 +878,10 @@ __device__ __forceinline__ bool donate_shallowest(const BkParams &pr, Sub &s, ui
       if (t) {
         const uint32_t k = w + mbcnt(m);
         if (kIPX) {
-          sXI[k] = s.XV[e];
-          for (uint32_t x = 0; x < W; ++x) sXR[(uint64_t)k * W + x] = s.XR[(uint64_t)e * W + x];
+          st_shared(sXI + k, s.XV[e]);
+          for (uint32_t x = 0; x < W; ++x) st_shared(sXR + (uint64_t)k * W + x, s.XR[(uint64_t)e * W + x]);
         } else {
-          sXI[k] = e;
+          st_shared(sXI + k, e);
         }
       }
       w += popc64(m);
@@ -1291,23 +1327,13 @@ __device__ __forceinline__ bool send_bits(const BkParams &pr, const Sub &s, uint
   const uint32_t rcv = claim_receiver(pr, wa.xq);
   if (rcv == kNone) return false;
   uint8_t *slot = pr.ring + (uint64_t)rcv * pr.slot_bytes;
-  if (L == 0) {
-    uint32_t *h = (uint32_t *)slot;
-    h[0] = s.root;
-    h[1] = rsize;
-    h[2] = s.p;
-    h[3] = W;
-    h[4] = 0;  // outside rows: set once they are packed
-    h[5] = kTaskBits;
-    *(uint64_t *)(slot + 24) = rmix;
-  }
   uint64_t *sp = (uint64_t *)(slot + pr.slot_oP);
   if (L < W) {
-    sp[L] = Pn;
-    sp[pr.slot_wmax + L] = Xn;
+    st_shared(sp + L, Pn);
+    st_shared(sp + pr.slot_wmax + L, Xn);
   }
-  wave_copy((uint32_t *)(slot + pr.slot_oS), s.S, s.p);
-  copy64((uint64_t *)(slot + pr.slot_oA), s.A, (uint64_t)s.p * W);
+  wave_copy<true>((uint32_t *)(slot + pr.slot_oS), s.S, s.p);
+  copy64<true>((uint64_t *)(slot + pr.slot_oA), s.A, (uint64_t)s.p * W);
   uint64_t *sXR = (uint64_t *)(slot + pr.slot_oXR);
   uint32_t qn = 0;
   for (uint64_t em = ballot(En != 0); em; em &= em - 1) {
@@ -1315,12 +1341,12 @@ __device__ __forceinline__ bool send_bits(const BkParams &pr, const Sub &s, uint
     const uint64_t ek = rdlane64(En, k);
     if ((ek >> L) & 1ull) {
       const uint64_t src = (uint64_t)(k * 64 + L) * W, dst = (uint64_t)(qn + mbcnt(ek)) * W;
-      for (uint32_t w = 0; w < W; ++w) sXR[dst + w] = ld64<kLX>(s.XR, src + w);
+      for (uint32_t w = 0; w < W; ++w) st_shared(sXR + dst + w, ld64<kLX>(s.XR, src + w));
     }
     qn += popc64(ek);
   }
-  if (L < (qn + 63) / 64) sp[2 * pr.slot_wmax + L] = full_word(qn);
-  if (L == 0) ((uint32_t *)slot)[4] = qn;
+  if (L < (qn + 63) / 64) st_shared(sp + 2 * pr.slot_wmax + L, full_word(qn));
+  put_header(slot, s.root, rsize, s.p, W, qn, kTaskBits, rmix);
   publish_task(pr, rcv);
   return true;
 }
@@ -2390,20 +2416,16 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
       clk.to(kBdQueue);
       if (!registered) registered = register_idle(pr, gw, wa.xq);
       if (registered) {
-        // relaxed poll (an acquire at agent scope would invalidate the CU's
-        // vector L1 on every poll, under the waves still at work); the
-        // acquire fence follows only once a task is in
-        const unsigned long long got = uniform64(
-            L == 0 ? __hip_atomic_load(&pr.mbox[(uint64_t)gw * kMboxStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                   : 0ull);
+        const unsigned long long got = uniform64(L == 0 ? ld_relaxed(&pr.mbox[(uint64_t)gw * kMboxStride]) : 0ull);
         if (got) {
           registered = false;
           backoff = 1;
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-          const uint32_t *h = (const uint32_t *)slot;
-          const uint32_t root = uniform(h[0]), rsize = uniform(h[1]), p = uniform(h[2]), W = uniform(h[3]),
-                         nx = uniform(h[4]), kind = uniform(h[5]);
-          const uint64_t rmix = uniform64(*(const uint64_t *)(slot + 24));
+          drain();
+          const uint64_t *h = (const uint64_t *)slot;
+          const uint64_t h0 = uniform64(ld_shared(h)), h1 = uniform64(ld_shared(h + 1)), h2 = uniform64(ld_shared(h + 2)),
+                         rmix = uniform64(ld_shared(h + 3));
+          const uint32_t root = (uint32_t)h0, rsize = (uint32_t)(h0 >> 32), p = (uint32_t)h1, W = (uint32_t)(h1 >> 32),
+                         nx = (uint32_t)h2, kind = (uint32_t)(h2 >> 32);
           if (kIPX && kind == kTaskBits) {
             const bool shape = p <= pr.slot_pmax && W == (p + 63) / 64 && nx <= pr.slot_xcap && nx <= kMaxXRows;
             if (shape)
@@ -2415,17 +2437,13 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
             if (okb) {
               const uint64_t *sp = (const uint64_t *)(slot + pr.slot_oP);
               if (L < W) {
-                P0 = sp[L];
-                X0 = sp[pr.slot_wmax + L];
+                P0 = ld_shared(sp + L);
+                X0 = ld_shared(sp + pr.slot_wmax + L);
               }
-              if (L < s.WX) E0 = sp[2 * pr.slot_wmax + L];
-              wave_copy(s.S, (const uint32_t *)(slot + pr.slot_oS), p);
-              const uint64_t *sA = (const uint64_t *)(slot + pr.slot_oA);
-              const uint64_t nA = (uint64_t)p * W;
-              copy64(s.A, sA, nA);
-              const uint64_t *sXR = (const uint64_t *)(slot + pr.slot_oXR);
-              const uint64_t nR = (uint64_t)nx * W;
-              copy64(s.XR, sXR, nR);
+              if (L < s.WX) E0 = ld_shared(sp + 2 * pr.slot_wmax + L);
+              wave_copy<false, true>(s.S, (const uint32_t *)(slot + pr.slot_oS), p);
+              copy64<false, true>(s.A, (const uint64_t *)(slot + pr.slot_oA), (uint64_t)p * W);
+              copy64<false, true>(s.XR, (const uint64_t *)(slot + pr.slot_oXR), (uint64_t)nx * W);
               s.p = p;
               fill_hash_terms(s);
             }
@@ -2466,22 +2484,18 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
           if (ok) {
             const uint64_t *sp = (const uint64_t *)(slot + pr.slot_oP);
             if (L < W) {
-              P0 = sp[L];
-              X0 = sp[pr.slot_wmax + L];
+              P0 = ld_shared(sp + L);
+              X0 = ld_shared(sp + pr.slot_wmax + L);
             }
-            wave_copy(s.S, (const uint32_t *)(slot + pr.slot_oS), p);
-            const uint64_t *sA = (const uint64_t *)(slot + pr.slot_oA);
-            const uint64_t nA = (uint64_t)p * W;
-            copy64(s.A, sA, nA);
+            wave_copy<false, true>(s.S, (const uint32_t *)(slot + pr.slot_oS), p);
+            copy64<false, true>(s.A, (const uint64_t *)(slot + pr.slot_oA), (uint64_t)p * W);
             const uint32_t *sXI = (const uint32_t *)(slot + pr.slot_oXI);
             if (kIPX) {
-              wave_copy(s.XV, sXI, nx);
-              const uint64_t *sXR = (const uint64_t *)(slot + pr.slot_oXR);
-              const uint64_t nR = (uint64_t)nx * W;
-              copy64(s.XR, sXR, nR);
+              wave_copy<false, true>(s.XV, sXI, nx);
+              copy64<false, true>(s.XR, (const uint64_t *)(slot + pr.slot_oXR), (uint64_t)nx * W);
               for (uint32_t i = L; i < nx; i += kWave) s.XL[i] = i;
             } else {
-              wave_copy(s.XL, sXI, nx);
+              wave_copy<false, true>(s.XL, sXI, nx);
             }
           }
           if (ok) {
