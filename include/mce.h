@@ -104,11 +104,14 @@ typedef struct mce_opts {
                               subproblems that need more than the cap run
                               in a second launch with larger arenas       */
   int stack_lds_levels;    /* BK frames kept in LDS before spilling to HBM  */
-  int donate_min_p;        /* donate a child only if |P| >= this (SZTH)     */
+  int donate_min_p;        /* donate a child only if |P| >= this (SZTH); the
+                              default, 10, with donate_age_us 0: automatic
+                              (20..33)                                      */
   int donate_check_nodes;  /* tree nodes between polls of the idle count    */
   int donate_age_us;       /* a task donates only after running this long
-                              (0 = 1000 us): short tasks finish sooner
-                              than a copy of their bit matrix pays back    */
+                              (0 = 50 us or 1 ms, as donate_min_p's): short
+                              tasks finish sooner than a copy of their bit
+                              matrix pays back                             */
   int split_heavy;         /* learned schedule at level 1, the variant per
                               subproblem: N > 0 runs every vertex predicted
                               above N tree nodes as its level-2 arc
@@ -134,9 +137,10 @@ typedef struct mce_opts {
                               the worker list, tasks outstanding and the
                               busy waves' node heartbeats); 0 = silent      */
   int lane_universe;       /* small-universe solver: a subtree whose P and X
-                              number at most this many members runs on one
-                              lane, 64 such subtrees per wave at a time
-                              (1..16; 0 = 16; -1 = never)                   */
+                              number at most this many members (and P at
+                              most 15) runs on one lane, 64 such subtrees
+                              per wave at a time (1..16; 0 = all that fit
+                              a lane, 15 of P and 48 of X; -1 = never)      */
 
   int schedule;            /* enum mce_schedule                              */
   const uint32_t *order;   /* MCE_SCHED_GIVEN: first-level vertex order      */

@@ -62,6 +62,10 @@ void fill_order_fields(const mce_graph *h, mce_result *res) {
 
 }  // namespace
 
+// donate_min_p of mce_opts_default; with the age at 0 it stands for the
+// engine's own thresholds.
+constexpr int kDefaultMinP = 10;
+
 int check_opts(const mce_opts *o) {
   if (o->level != MCE_L1 && o->level != MCE_L2) return set_error(MCE_EINVAL, "level must be MCE_L1 or MCE_L2");
   if (o->induced != MCE_IP && o->induced != MCE_IPX) return set_error(MCE_EINVAL, "induced must be MCE_IP or MCE_IPX");
@@ -104,7 +108,7 @@ void mce_opts_default(mce_opts *o) {
   o->worklist = MCE_NOWL;
   o->task = MCE_TASK_MCE;
   o->device = 0;
-  o->donate_min_p = 10;
+  o->donate_min_p = kDefaultMinP;
   o->schedule = MCE_SCHED_PLAIN;
 }
 
@@ -408,18 +412,30 @@ static int count_impl(mce_graph *h, const mce_opts *opts, mce_result *res, bool 
   cfg.stack_lds_levels = (uint32_t)opts->stack_lds_levels;
   cfg.donate_min_p = (uint32_t)opts->donate_min_p;
   cfg.donate_check_nodes = opts->donate_check_nodes ? (uint32_t)opts->donate_check_nodes : 64;
-  cfg.donate_age_us = opts->donate_age_us ? (uint32_t)opts->donate_age_us : 1000;
   cfg.capture = capture || opts->graph_launch;
   cfg.small_max = opts->small_universe < 0 ? 0u : opts->small_universe ? (uint32_t)opts->small_universe : 64u;
-  cfg.lane_max = opts->lane_universe < 0 ? 0u : opts->lane_universe ? (uint32_t)opts->lane_universe : 16u;
+  cfg.lane_max = opts->lane_universe < 0 ? 0u : opts->lane_universe ? (uint32_t)opts->lane_universe : kLaneAuto;
   cfg.hbm_bytes = (uint64_t)opts->hbm_arena_bytes;
   cfg.watchdog_us = (uint32_t)opts->watchdog_us;
   cfg.progress_s = (uint32_t)opts->progress_s;
-  if (heavy_tail && !opts->donate_age_us) {
-    // thresholds set from the cost model: with a predicted heavy tail only
-    // long-running tasks donate (a donation copies the donor's bit matrix;
-    // frequent small donations cost more than they balance)
-    cfg.donate_age_us = 10000;
+  // Worker list, thresholds left to the engine. A donation copies the donor's
+  // bit matrix, some 10 us; what it is worth depends on how fast the donor
+  // would have been. Enumeration in ms for a task age of 50 us / 1 ms and a
+  // child of at least |P| members (IPX; R-MAT 14 | Chung-Lu 2^17, no model):
+  //   lane solver     |P| 28   21.5 / 26.5 | 24.2 / 17.8
+  //                   |P| 33   21.4 / 27   | 18.1 / 15.4
+  //   no lane solver  |P| 28   -           | 35.7 / 21.5   (R-MAT 12: 5.5 / 6.1)
+  // IP solves subtrees on the list path, two times as slow a node
+  // (R-MAT 13, 50 us): |P| 10 9.5, 16 5.2, 20 3.5, 24 5.2, 28 8.1; R-MAT 12
+  // arcs 9.4, 5.5, 5.9, 8.9, 16.9. With a predicted heavy tail (Chung-Lu
+  // 2^18) 50 us 76.0, 400 us 73.0, 1 ms 72.1, 3 ms 73.5. From |P| 33 on the
+  // small-universe solver does not take a child whole.
+  cfg.donate_auto = opts->donate_age_us == 0 && opts->donate_min_p == kDefaultMinP;
+  const bool lanes = cfg.ipx && cfg.lane_max && cfg.small_max;
+  cfg.donate_age_us = opts->donate_age_us ? (uint32_t)opts->donate_age_us : 1000;
+  if (cfg.donate_auto) {
+    cfg.donate_age_us = heavy_tail || (cfg.ipx && !lanes) ? 1000 : 50;
+    cfg.donate_min_p = !cfg.ipx ? 20 : lanes ? 33 : 28;
   }
   BkOut out;
   const bool want_waves = opts->task == MCE_TASK_LB_EVAL || opts->task == MCE_TASK_DONOR_EVAL ||

@@ -73,6 +73,10 @@ enum Acc : uint32_t {
 // statistics with the lane solver compiled in (kept out of the other
 // instances, whose register allocation it would otherwise share).
 enum Stat : int { kStatNone = 0, kStatLb = 1, kStatDonor = 2, kStatBd = 3, kStatLane = 4 };
+// Kernel instances that solve in functions of their own (see "functions of
+// their own" below): those of the bitmap path without statistics. The IP
+// instances only have the list path, whose code stays in the kernel.
+constexpr bool fn_of(bool ipx, int stat) { return ipx && (stat == kStatNone || stat == kStatLane); }
 constexpr bool lane_of(int stat) { return stat == kStatLane; }
 enum Bd : int { kBdOther = 0, kBdInduced, kBdQueue, kBdPivot, kBdSetOps, kBdMaximal, kBdBranch };
 
@@ -81,6 +85,7 @@ enum Bd : int { kBdOther = 0, kBdInduced, kBdQueue, kBdPivot, kBdSetOps, kBdMaxi
 // not contend for one line.
 constexpr uint32_t kQueues = 8;
 // Word kCtlProgress (a line of its own) counts heartbeats of busy waves.
+constexpr unsigned long long kMboxTask = 1, kMboxDone = 2;
 constexpr uint32_t kCtlProgress = 0, kCtlOutstanding = 16, kCtlQueues = 32, kCtlWords = kCtlQueues + 16 * kQueues;
 // Mailbox words of the waves, each on its own 128-byte line.
 constexpr uint32_t kMboxStride = 16;
@@ -137,7 +142,7 @@ struct BkParams {
   uint8_t *ring;           // task slots, one per wave
   uint32_t ring_cap;       // idle-queue capacity (= waves)
   uint32_t *idle_ids;      // idle queue entries: wave ids
-  unsigned long long *mbox;  // per-wave mailbox: 1 once a task is in the wave's slot
+  unsigned long long *mbox;  // per-wave mailbox: kMboxTask once a task is in the wave's slot, kMboxDone at the end
   uint64_t slot_bytes;       // task slot per wave (pr.ring + wave * slot_bytes)
   uint32_t slot_pmax;  // largest donor |S|
   uint32_t slot_wmax;
@@ -146,19 +151,23 @@ struct BkParams {
   uint32_t donate_min_p;
   uint32_t donate_check;
   uint64_t donate_age;  // 100 MHz realtime ticks a task runs before it may donate
+  uint64_t poll_ticks;  // realtime ticks between looks at the idle queues
   uint32_t small_max;   // nodes with P + X + outside rows <= this go to the small-universe solver
   uint32_t small_pmax;  // ... and, with the worker list, |P| <= this
   uint64_t watchdog_ticks;  // idle time without global progress before the kernel gives up
   // pinned host words the kernel mirrors its progress into while it runs
   // (word 0: a recent ticket claimed, word 1: heartbeats); nullable
   unsigned long long *host_progress;
-  // lane solver (ls_max = 0: off): largest member count, byte offset of the
-  // waves' LDS regions in the workgroup's LDS, hash-term slots of every wave
+  // lane solver (ls_max = 0: off): largest member count, the waves' regions
   uint32_t ls_max;
-  uint32_t ls_off;
-  uint64_t *ls_h;
+  uint32_t ls_off;  // byte offsets of the waves' LDS parts: found cliques, hand-over blocks
+  uint32_t io_off;
+  uint8_t *ls;
   uint64_t *cover;  // hub row filter: 64 words per wave
 };
+
+// The workgroup's histogram bins in LDS, typed as such.
+typedef __attribute__((address_space(3))) unsigned long long lds_ull;
 
 // Posts a progress value to pinned host memory (a system-scope vector store;
 // the host polls it while the persistent launch holds every CU, when a copy
@@ -189,6 +198,7 @@ struct Sub {
   const uint64_t *rp;
   const uint64_t *split;
   uint64_t *cover;  // hub row filter: the wave's 64 union words (device memory)
+  uint64_t t0;      // realtime at which the subproblem was taken up
 };
 
 struct WaveAcc {
@@ -196,17 +206,23 @@ struct WaveAcc {
   uint32_t max_size = 0;
   uint64_t sub_cliques = 0;
   int32_t budget = 0;
-  uint64_t last_poll = 0;
-  uint64_t last_beat = 0;  // tree nodes at the last heartbeat
+  uint64_t last_poll = 0;  // nodes at the last poll
+  uint64_t next_poll = 0;  // realtime before which the idle queues are not looked at
+  uint64_t poll_wait = 1;
+  uint64_t last_beat = 0;  // tree nodes (lane solver's included) at the last heartbeat
   uint32_t xq = 0;      // this wave's idle queue (its XCD)
   uint32_t peek = 0;    // another queue sampled at the next poll
   uint64_t t_task = 0;  // realtime at the start of the current task
-  // lane solver: queued subtrees, their largest member count, this wave's
-  // LDS region and hash-term slots
-  uint32_t ls_n = 0, ls_u = 0, ls_lds = 0;
-  uint64_t *ls_h = nullptr;
+  // lane solver: queued subtrees, the most P and X members among them, this
+  // wave's region; what its runs found (their labels go to the subtrees'
+  // roots, so they stay out of the running subproblem's counts)
+  uint32_t ls_n = 0, ls_p = 0, ls_x = 0, ls_lds = 0;
+  uint32_t io = 0;  // LDS address of the wave's hand-over block
+  uint8_t *ls = nullptr;
+  uint64_t ls_nodes = 0, ls_count = 0;
 };
 
+typedef const __attribute__((address_space(4))) BkParams ConstParams;
 template <int kStat>
 struct Clock {
   uint64_t acc[7];
@@ -453,7 +469,7 @@ __device__ __forceinline__ Region pool_take(const Pool &pl, uint32_t want, uint3
   return r;
 }
 
-__device__ __forceinline__ void pool_put(const Pool &pl, const Region &r) {
+__device__ __forceinline__ void pool_give(const Pool &pl, const Region &r) {
   if (r.gk && lane_id() == 0) {
     pool_lock(pl.lock);
     pool_mark(pl, r.g0, r.gk, false);
@@ -464,19 +480,59 @@ __device__ __forceinline__ void pool_put(const Pool &pl, const Region &r) {
 // pool_take that waits (up to about a millisecond) for at least `need` bytes
 // when the pool could hold them: a subproblem run from HBM costs far more
 // than the wait, and the waves holding LDS never wait, so space comes free.
-__device__ __forceinline__ Region pool_take_wait(const Pool &pl, uint32_t want, uint32_t mid, uint32_t low,
+__device__ __forceinline__ Region pool_take_wait_in(const Pool &pl, uint32_t want, uint32_t mid, uint32_t low,
                                                  uint32_t need) {
   Region r = pool_take(pl, want, mid, low);
   if (r.bytes >= need || need > pl.ngran * kGranule) return r;
   uint32_t backoff = 1;
   for (uint32_t t = 0; t < 24; ++t) {
-    pool_put(pl, r);
+    pool_give(pl, r);
     for (uint32_t z = 0; z < backoff; ++z) __builtin_amdgcn_s_sleep(32);
     backoff = min(backoff * 2, 32u);
     r = pool_take(pl, want, mid, low);
     if (r.bytes >= need) return r;
   }
   return r;
+}
+// Both also as functions, for the kernel's many places (the search for a run
+// of free granules alone is inlined six times in a taking); mask: the LDS
+// address of the pool's words.
+typedef __attribute__((address_space(3))) uint8_t lds_u8;
+__device__ __forceinline__ Pool pool_at(uint32_t mask, uint32_t ngran) {
+  uint8_t *at = (uint8_t *)(lds_u8 *)(uintptr_t)uniform(mask);
+  Pool pl;
+  pl.mask = (uint64_t *)at;
+  pl.lock = (uint32_t *)(at + 8 * kPoolWords);
+  pl.base = at + kPoolHeader;
+  pl.ngran = uniform(ngran);
+  return pl;
+}
+__device__ __noinline__ __attribute__((not_tail_called)) uint64_t pool_take_fn(uint32_t mask, uint32_t ngran, uint32_t want,
+                                                                               uint32_t mid, uint32_t low, uint32_t need) {
+  const Region r =
+      pool_take_wait_in(pool_at(mask, ngran), uniform(want), uniform(mid), uniform(low), uniform(need));
+  return (uint64_t)r.gk << 32 | r.g0;
+}
+__device__ __noinline__ __attribute__((not_tail_called)) void pool_put_fn(uint32_t mask, uint32_t ngran, uint32_t g0,
+                                                                          uint32_t gk) {
+  pool_give(pool_at(mask, ngran), Region{nullptr, 0, uniform(g0), uniform(gk)});
+}
+template <bool kFn>
+__device__ __forceinline__ Region pool_take_wait(const Pool &pl, uint32_t want, uint32_t mid, uint32_t low,
+                                                 uint32_t need) {
+  if constexpr (!kFn) return pool_take_wait_in(pl, want, mid, low, need);
+  const uint64_t got = uniform64(pool_take_fn((uint32_t)(uintptr_t)pl.mask, pl.ngran, want, mid, low, need));
+  Region r;
+  r.g0 = (uint32_t)got;
+  r.gk = (uint32_t)(got >> 32);
+  r.ptr = pl.base + (r.gk ? (uint64_t)r.g0 * kGranule : 0);
+  r.bytes = r.gk * kGranule;
+  return r;
+}
+template <bool kFn>
+__device__ __forceinline__ void pool_put(const Pool &pl, const Region &r) {
+  if constexpr (!kFn) pool_give(pl, r);
+  else if (r.gk) pool_put_fn((uint32_t)(uintptr_t)pl.mask, pl.ngran, r.g0, r.gk);
 }
 
 __device__ __forceinline__ const uint64_t *row_of(const Sub &s, uint32_t piv) {
@@ -596,14 +652,14 @@ __device__ __forceinline__ uint32_t xe_partition(const Sub &s, uint32_t len, uin
   return kept;
 }
 
-__device__ __forceinline__ void report(const BkParams &pr, unsigned long long *hist_lds, WaveAcc &wa, uint32_t size,
+__device__ __forceinline__ void report(const BkParams &pr, lds_ull *hist_lds, WaveAcc &wa, uint32_t size,
                                        uint64_t mix) {
   wa.count++;
   wa.sub_cliques++;
   wa.hash += clique_hash(mix, size);
   wa.max_size = max(wa.max_size, size);
   if (lane_id() == 0) {
-    if (size < pr.hist_lds) atomicAdd(&hist_lds[size], 1ull);
+    if (size < pr.hist_lds) __hip_atomic_fetch_add(&hist_lds[size], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     else atomicAdd(&pr.hist[min(size, pr.hist_len - 1)], 1ull);
   }
 }
@@ -724,8 +780,8 @@ __device__ __forceinline__ uint32_t queue_len(const BkParams &pr, uint32_t q) {
 
 // Progress signal of a busy wave for the idle waves' watchdog.
 __device__ __forceinline__ void heartbeat(const BkParams &pr, WaveAcc &wa) {
-  if (wa.nodes - wa.last_beat >= kBeatNodes) {
-    wa.last_beat = wa.nodes;
+  if (wa.nodes + wa.ls_nodes - wa.last_beat >= kBeatNodes) {
+    wa.last_beat = wa.nodes + wa.ls_nodes;
     if (lane_id() == 0) {
       const unsigned long long b = atomicAdd(pr.ctl + kCtlProgress, 1ull);
       if (pr.host_progress) post_progress(pr.host_progress + 1, b + 1);
@@ -745,15 +801,39 @@ __device__ __forceinline__ int32_t donation_budget(const BkParams &pr, WaveAcc &
   return (int32_t)uniform((uint32_t)b);
 }
 
-// Takes an idle wave off the idle queues (this XCD's first) for a donation
+// A busy wave's poll, every donate_check nodes: its heartbeat, and from
+// donate_age on, at most once every poll_ticks, a look at the idle queues
+// (loads past the L2, some microseconds).
+__device__ __forceinline__ void poll_idle(const BkParams &pr, WaveAcc &wa) {
+  const uint64_t nodes = wa.nodes + wa.ls_nodes;
+  if (nodes - wa.last_poll < pr.donate_check) return;
+  wa.last_poll = nodes;
+  heartbeat(pr, wa);
+  const uint64_t now = __builtin_amdgcn_s_memrealtime();
+  wa.budget = 0;
+  if (now - wa.t_task < pr.donate_age || now < wa.next_poll) return;
+  wa.budget = donation_budget(pr, wa);
+  // nobody idle: look half as often each time, down to every 32 poll_ticks
+  // (thousands of busy waves on the queues' 16 lines keep the idle ones from
+  // getting on them)
+  wa.poll_wait = wa.budget ? pr.poll_ticks : min(2 * wa.poll_wait, 32 * pr.poll_ticks);
+  wa.next_poll = now + wa.poll_wait;
+}
+// No child to give, or nobody left to take it: the next look waits longer.
+__device__ __forceinline__ void no_donation(const BkParams &pr, WaveAcc &wa) {
+  wa.budget = 0;
+  wa.next_poll += 3 * pr.poll_ticks;
+}
+
+// Takes an idle wave off the two queues last looked at (this XCD's first) for a donation
 // and counts the task as outstanding; returns that wave's id (its slot
 // receives the task) or kNone.
-__device__ __forceinline__ uint32_t claim_receiver(const BkParams &pr, uint32_t xq) {
+__device__ __forceinline__ uint32_t claim_receiver(const BkParams &pr, const WaveAcc &wa) {
   uint32_t r = kNone;
   if (lane_id() == 0) {
-    for (uint32_t i = 0; i < kQueues && r == kNone; ++i) {
-      const uint32_t q = (xq + i) % kQueues;
-      if (i && queue_len(pr, q) == 0) continue;
+    for (uint32_t i = 0; i < 2 && r == kNone; ++i) {
+      const uint32_t q = i ? wa.peek : wa.xq;
+      if (i && q == wa.xq) break;
       const unsigned long long pos = ring_claim_pop(pr, q);
       if (pos != kNoSlot) {
         const uint64_t at = (uint64_t)q * pr.ring_cap + pos % pr.ring_cap;
@@ -783,24 +863,34 @@ __device__ __forceinline__ void put_header(uint8_t *slot, uint32_t root, uint32_
 // Hands the task written into receiver r's slot over to it.
 __device__ __forceinline__ void publish_task(const BkParams &pr, uint32_t r) {
   drain();  // the slot is written
-  if (lane_id() == 0) st_shared(&pr.mbox[(uint64_t)r * kMboxStride], 1ull);
+  if (lane_id() == 0) st_shared(&pr.mbox[(uint64_t)r * kMboxStride], kMboxTask);
 }
 
-// Puts this idle wave on its XCD's idle queue (its mailbox cleared first);
-// false when the queue's tail was too contended this time.
+// Puts this idle wave on its XCD's idle queue (its mailbox is empty); false when the queue's tail was too contended this time.
 __device__ __forceinline__ bool register_idle(const BkParams &pr, uint32_t gw, uint32_t xq) {
   unsigned long long pos = kNoSlot;
   if (lane_id() == 0) {
-    st_shared(&pr.mbox[(uint64_t)gw * kMboxStride], 0ull);
     pos = ring_claim_push(pr, xq);
     if (pos != kNoSlot) {
       const uint64_t at = (uint64_t)xq * pr.ring_cap + pos % pr.ring_cap;
       st_shared(&pr.idle_ids[at], gw);
-      drain();  // mailbox and id are written before the entry is published
+      drain();  // the id is written before the entry is published
       st_shared(&pr.seq[at], pos + 1);
     }
   }
   return uniform64(pos) != kNoSlot;
+}
+
+// Takes n tasks off the outstanding count. The wave that takes the last one
+// tells all others through their mailboxes: on their own they look at the
+// count every 16th poll only, some 0.2 ms apart once they have waited long
+// (worker-list launches in ms: 301 block-model graphs 1.77 -> 1.23, R-MAT 12
+// (ef 8) 1.53 -> 1.13, G(4,096, deg 20) 0.44 -> 0.34).
+__device__ __forceinline__ void tasks_done(const BkParams &pr, uint32_t n) {
+  unsigned long long left = 1;
+  if (lane_id() == 0) left = atomicSub(pr.ctl + kCtlOutstanding, (unsigned long long)n) - n;
+  if (uniform64(left) != 0) return;
+  for (uint32_t i = lane_id(); i < pr.ring_cap; i += kWave) st_shared(&pr.mbox[(uint64_t)i * kMboxStride], kMboxDone);
 }
 
 // Publishes the next child of the shallowest frame that still has one, when
@@ -852,7 +942,7 @@ __device__ __forceinline__ bool donate_shallowest(const BkParams &pr, Sub &s, ui
       nx += popc64(ballot(i < xej && xe_adj<kIPX>(s, s.XL[i], c, nb, nlen)));
     }
     if (nx > pr.slot_xcap || hbm_need(s.p, nx, kIPX) > pr.hbm_bytes) continue;
-    const uint32_t rcv = claim_receiver(pr, wa.xq);
+    const uint32_t rcv = claim_receiver(pr, wa);
     if (rcv == kNone) return false;
     uint8_t *slot = pr.ring + (uint64_t)rcv * pr.slot_bytes;
     put_header(slot, s.root, s.rsize + j + 1, s.p, W, nx, kTaskList, mixj + splitmix64(s.S[c]));
@@ -907,7 +997,7 @@ __device__ __forceinline__ bool donate_shallowest(const BkParams &pr, Sub &s, ui
 
 // Runs BK from the root state (P, X) of an arena that `build` has filled.
 template <bool kIPX, bool kWL, int kStat>
-__device__ __forceinline__ void bk_solve(const BkParams &pr, Sub &s, uint64_t cP, uint64_t cX, unsigned long long *hist_lds,
+__device__ __forceinline__ void bk_solve(const BkParams &pr, Sub &s, uint64_t cP, uint64_t cX, lds_ull *hist_lds,
                          WaveAcc &wa, Clock<kStat> &clk) {
   const uint32_t L = lane_id(), W = s.W;
   const bool act = L < W;
@@ -921,17 +1011,11 @@ __device__ __forceinline__ void bk_solve(const BkParams &pr, Sub &s, uint64_t cP
   uint32_t d = 0;
   while (true) {
     if constexpr (kWL) {
-      if (wa.nodes - wa.last_poll >= pr.donate_check) {
-        wa.last_poll = wa.nodes;
-        heartbeat(pr, wa);
-        clk.to(kBdQueue);
-        // only a task that has run for a while gives work away
-        wa.budget = __builtin_amdgcn_s_memrealtime() - wa.t_task >= pr.donate_age ? donation_budget(pr, wa) : 0;
-      }
+      clk.to(kBdQueue);
+      poll_idle(pr, wa);
       if (wa.budget > 0) {
-        clk.to(kBdQueue);
         if (donate_shallowest<kIPX>(pr, s, d, cP, cX, piv, xe, mix, wa)) wa.budget--;
-        else wa.budget = 0;
+        else no_donation(pr, wa);
       }
     }
     clk.to(kBdSetOps);
@@ -1125,19 +1209,25 @@ __device__ __forceinline__ void clear_cover(uint64_t *cover) {
 }
 
 // Number of rows keep_chunk keeps from the q vertices in ids, for any q.
-__device__ __forceinline__ uint32_t live_count(const BkParams &pr, const uint32_t *S, uint32_t p, const uint32_t *ids,
-                                               uint32_t q, uint64_t *cover) {
+__device__ __noinline__ __attribute__((not_tail_called)) uint32_t live_count_fn(ConstParams *kargs, const uint32_t *S,
+                                                                                uint32_t p, const uint32_t *ids, uint32_t q,
+                                                                                uint64_t *cover) {
+  const BkParams &pr = *(const BkParams *)(ConstParams *)uniform64((uint64_t)kargs);
+  p = uniform(p);
+  q = uniform(q);
   uint32_t n = 0;
   clear_cover(cover);
   for (uint32_t b = 0; b < q; b += kWave) n += popc64(keep_chunk(pr, S, p, ids, q, b, cover));
   return n;
 }
 
-__device__ __forceinline__ uint64_t live_rows(const BkParams &pr, const uint32_t *S, uint32_t p, const uint32_t *ids,
-                                              uint32_t q, uint32_t &nkeep) {
+__device__ __noinline__ __attribute__((not_tail_called)) uint64_t live_rows_fn(ConstParams *kargs, const uint32_t *S,
+                                                                               uint32_t p, const uint32_t *ids, uint32_t q) {
+  const BkParams &pr = *(const BkParams *)(ConstParams *)uniform64((uint64_t)kargs);
+  p = uniform(p);
+  q = uniform(q);
   const uint32_t L = lane_id();
   uint64_t keep = 0;
-  nkeep = 0;
   for (uint32_t b = 0, k = 0; b < q; b += kWave, ++k) {
     const uint32_t i = b + L;
     bool any = false;
@@ -1151,14 +1241,65 @@ __device__ __forceinline__ uint64_t live_rows(const BkParams &pr, const uint32_t
     }
     const uint64_t m = ballot(any);
     if (L == k) keep = m;
-    nkeep += popc64(m);
   }
+  return keep;
+}
+
+__device__ __forceinline__ uint32_t live_count(const uint32_t *S, uint32_t p, const uint32_t *ids, uint32_t q,
+                                               uint64_t *cover) {
+  return uniform(live_count_fn((ConstParams *)__builtin_amdgcn_kernarg_segment_ptr(), S, p, ids, q, cover));
+}
+__device__ __forceinline__ uint64_t live_rows(const uint32_t *S, uint32_t p, const uint32_t *ids, uint32_t q,
+                                              uint32_t &nkeep) {
+  const uint64_t keep = live_rows_fn((ConstParams *)__builtin_amdgcn_kernarg_segment_ptr(), S, p, ids, q);
+  nkeep = wave_sum(popc64(keep));
   return keep;
 }
 
 // Keep mask of all q rows (lane k: rows 64k..64k+63).
 __device__ __forceinline__ uint64_t all_rows(uint32_t q) { return full_word(q); }
 
+// ---- functions of their own -----------------------------------------------
+// The kernel's places that set a subproblem up and solve it call functions:
+// with everything inlined a kernel was 119,000 instructions, the solver
+// shared its registers with all that surrounds it, and what bounded a small
+// subproblem was the scratch memory its registers were spilled to (500 bytes
+// a lane, 32 KB a wave and subproblem). `kargs` is the kernel's argument
+// segment, whose first argument is pr; s goes through the wave's hand-over
+// block in LDS (address wa.io) once a subproblem, the wave's totals stay
+// there, and both are read back as uniform values. not_tail_called lets the
+// compiler see which registers a function leaves alone (otherwise each call
+// saved and restored 54 of them). Enumeration in ms, everything inlined but
+// the solvers -> now: G(4,096, deg 20) 0.175 -> 0.10, G(50,000, deg 40) 1.56
+// -> 1.14, 301 block-model graphs of 64..300 1.22 -> 0.79, of 400..500 4.26
+// -> 2.73, R-MAT 12 (ef 8) 0.53 -> 0.48.
+struct Handover {
+  Sub s;
+  WaveAcc w;
+};
+typedef __attribute__((address_space(3))) Handover LdsHandover;
+constexpr uint32_t kHandoverBytes = (sizeof(Handover) + 15) / 16 * 16;
+__device__ __forceinline__ LdsHandover *handover(uint32_t io) { return (LdsHandover *)(uintptr_t)io; }
+// Word copies between registers and the block (all lanes hold and write the
+// same values).
+template <class T>
+__device__ __forceinline__ void lds_put(__attribute__((address_space(3))) T *to, const T &v) {
+  static_assert(sizeof(T) % 8 == 0, "whole words");
+  uint64_t t[sizeof(T) / 8];
+  __builtin_memcpy(t, &v, sizeof(T));
+#pragma unroll
+  for (uint32_t i = 0; i < sizeof(T) / 8; ++i) ((lds_u64 *)to)[i] = t[i];
+}
+// (read back as uniform values)
+template <class T>
+__device__ __forceinline__ T lds_get(const __attribute__((address_space(3))) T *from) {
+  uint64_t t[sizeof(T) / 8];
+#pragma unroll
+  for (uint32_t i = 0; i < sizeof(T) / 8; ++i) t[i] = uniform64(((const lds_u64 *)from)[i]);
+  T v;
+  __builtin_memcpy(&v, t, sizeof(T));
+  return v;
+}
 // Builds A over S and the kept outside rows (keep: mask from live_rows over
 // the q0 vertices in `ids`; s.q = their count), numbered in order; returns
 // this lane's word of the initial outside-row set (all kept rows).
@@ -1204,6 +1345,13 @@ __device__ __forceinline__ uint64_t build_bits(const BkParams &pr, Sub &s, const
   fill_hash_terms(s);
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
   return full_word(q);
+}
+
+__device__ __noinline__ __attribute__((not_tail_called)) uint64_t build_bits_fn(ConstParams *kargs, uint32_t io, const uint32_t *ids, uint32_t q0,
+                                               uint64_t keep, uint32_t filter) {
+  const BkParams &pr = *(const BkParams *)(ConstParams *)uniform64((uint64_t)kargs);
+  Sub s = lds_get(&handover(uniform(io))->s);
+  return build_bits(pr, s, (const uint32_t *)uniform64((uint64_t)ids), uniform(q0), keep, uniform(filter) != 0);
 }
 
 // Pivot over P|X (index order) then the outside rows in E (row order): the
@@ -1324,7 +1472,7 @@ template <bool kLX>
 __device__ __forceinline__ bool send_bits(const BkParams &pr, const Sub &s, uint32_t rsize, uint64_t rmix,
                                           uint64_t Pn, uint64_t Xn, uint64_t En, WaveAcc &wa) {
   const uint32_t L = lane_id(), W = s.W;
-  const uint32_t rcv = claim_receiver(pr, wa.xq);
+  const uint32_t rcv = claim_receiver(pr, wa);
   if (rcv == kNone) return false;
   uint8_t *slot = pr.ring + (uint64_t)rcv * pr.slot_bytes;
   uint64_t *sp = (uint64_t *)(slot + pr.slot_oP);
@@ -1354,7 +1502,7 @@ __device__ __forceinline__ bool send_bits(const BkParams &pr, const Sub &s, uint
 // Publishes the next child of the shallowest frame with a large enough child
 // (bitmap path): the donor's S, A and outside rows plus the child's P, X, E.
 template <bool kLA, bool kLX>
-__device__ __forceinline__ bool donate_bits(const BkParams &pr, Sub &s, uint32_t d, uint64_t &cP, uint64_t &cX, uint64_t cE,
+__device__ __forceinline__ bool donate_bits(const BkParams &pr, const Sub &s, uint32_t d, uint64_t &cP, uint64_t &cX, uint64_t cE,
                             uint32_t cpiv, uint64_t cmix, WaveAcc &wa) {
   const uint32_t L = lane_id(), W = s.W, WX = s.WX;
   const bool act = L < W;
@@ -1431,17 +1579,17 @@ struct CliqueBuf {
   uint32_t size = 0, n = 0;
 };
 
-__device__ __forceinline__ void flush_cliques(const BkParams &pr, unsigned long long *hist_lds, CliqueBuf &cb) {
+__device__ __forceinline__ void flush_cliques(const BkParams &pr, lds_ull *hist_lds, CliqueBuf &cb) {
   if (lane_id() < cb.n) {
     cb.hacc += clique_hash(cb.mix, cb.size);
-    if (cb.size < pr.hist_lds) atomicAdd(&hist_lds[cb.size], 1ull);
+    if (cb.size < pr.hist_lds) __hip_atomic_fetch_add(&hist_lds[cb.size], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     else atomicAdd(&pr.hist[min(cb.size, pr.hist_len - 1)], 1ull);
   }
   cb.n = 0;
 }
 
 // (the caller flushes before the buffer can overflow)
-__device__ __forceinline__ void keep_clique(const BkParams &pr, unsigned long long *hist_lds, WaveAcc &t,
+__device__ __forceinline__ void keep_clique(const BkParams &pr, lds_ull *hist_lds, WaveAcc &t,
                                             CliqueBuf &cb, uint32_t size, uint64_t mix) {
   cb.mix = wrlane64(cb.mix, cb.n, mix);
   cb.size = wrlane(cb.size, cb.n, size);
@@ -1466,10 +1614,13 @@ __device__ __forceinline__ uint64_t wave_add64(uint64_t v) {
 // 16..40 on R-MAT 14, Chung-Lu 2^19 and a 32-graph SBM batch.
 constexpr uint32_t kSmallMaxPWl = 32;
 template <bool kWL>
-__device__ __forceinline__ bool small_ok(const BkParams &pr, uint64_t P, uint64_t X, uint64_t E) {
-  const uint32_t np = popc64(P);
-  if (kWL && wave_sum(np) > pr.small_pmax) return false;
-  return wave_sum(np + popc64(X) + popc64(E)) <= pr.small_max;
+__device__ __forceinline__ bool small_ok(const BkParams &pr, uint64_t P, uint64_t X, uint64_t E, uint32_t &np,
+                                         uint32_t &nx) {
+  // both counts in one reduction (each is at most 64 x 192 < 2^16)
+  const uint32_t n = wave_sum(popc64(P) | (popc64(X) + popc64(E)) << 16);
+  np = n & 0xFFFFu;
+  nx = n >> 16;
+  return np + nx <= pr.small_max && (!kWL || np <= pr.small_pmax);
 }
 
 // Mask width of the small-universe solver's loop: a universe of at most 32
@@ -1487,6 +1638,7 @@ struct MaskOps<uint32_t> {
   // as a lane mask: lanes 32..63 hold no member
   __device__ static uint64_t lanes(uint32_t m) { return m; }
   __device__ static uint32_t wr(uint32_t f, uint32_t l, uint32_t v) { return wrlane(f, l, v); }
+  __device__ static uint32_t permute(uint32_t to, uint32_t v) { return (uint32_t)__builtin_amdgcn_ds_permute((int)to, (int)v); }
 };
 template <>
 struct MaskOps<uint64_t> {
@@ -1495,107 +1647,106 @@ struct MaskOps<uint64_t> {
   __device__ static uint64_t rd(uint64_t v, uint32_t l) { return rdlane64(v, l); }
   __device__ static uint64_t lanes(uint64_t m) { return m; }
   __device__ static uint64_t wr(uint64_t f, uint32_t l, uint64_t v) { return wrlane64(f, l, v); }
+  __device__ static uint64_t permute(uint32_t to, uint64_t v) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_permute((int)to, (int)(uint32_t)v);
+    return (uint64_t)(uint32_t)__builtin_amdgcn_ds_permute((int)to, (int)(v >> 32)) << 32 | lo;
+  }
 };
 
 // ---------------------------------------------------------------------------
-// Lane solver: subtrees whose P and X number at most kLsMax members run one
-// per lane, up to kLsSlots of them at a time. The small-universe solver
-// queues such a subtree (ls_put) instead of descending into it: the members
-// are renumbered 0..k-1 in their order, so pivots (largest |P & N(u)|, ties to
-// the lowest member) and child order (lowest member first) are unchanged, and
-// the lane visits the nodes the wave would have visited. A full queue, and
-// the end of every bitmap subproblem, runs the queue (ls_run).
+// Lane solver: subtrees with at most kLsP members in P and kLsX in X run one
+// per lane, kLsSlots at a time. The small-universe solver queues such a
+// subtree (ls_put), whole if its root fits, instead of working it off on the
+// wave; a full queue and the end of a wave's work run the queue (ls_run), so
+// that subtrees of many small subproblems share a run.
 //
-// Per wave: in LDS only the slots' rows (16-bit masks over the members, read
-// at every node; 2 KiB, so that the bit matrices' LDS pool keeps most of its
-// room); in device memory the members' hash terms (kLsMax 64-bit words per
-// slot), one 16-byte header per slot (P | k << 16, |R| at the subtree's root,
-// R's hash sum) and kLsLevels frames per slot ((P | X << 16), level-major so
-// that lanes at one depth touch consecutive words).
-constexpr uint32_t kLsMax = 16, kLsSlots = 64;
-// A pushed level has |P| >= 3 and every level has one member fewer in P than
-// its parent, so at most kLsMax - 3 levels are pushed.
-constexpr uint32_t kLsLevels = kLsMax - 3;
-constexpr uint32_t kLsBytes = kLsSlots * kLsMax * 2;  // LDS per wave
-constexpr uint32_t kLsHdrOff = kLsSlots * kLsMax * 8, kLsFrOff = kLsHdrOff + kLsSlots * 16,
-                   kLsGlobalBytes = kLsFrOff + kLsLevels * kLsSlots * 4;  // device memory per wave
-// the small-universe solver starts only with this many free slots
-constexpr uint32_t kLsReserve = 16;
+// What bounds the wave-wide loop is instructions: about 120 a node, for the
+// 24 members an average block-model universe has on 64 lanes. Here a step,
+// one node on every busy lane, is about 300 instructions. A node is decided
+// by which members each member of P sees: column r, of P's member r, holds a
+// bit for every member, P's at bits 0..15 and X's from bit 16 on (two words,
+// the second for X's members 16..47). A child's P' and X' are one AND with
+// its column. The pivot scores |P' & N(u)| of all members at once are a sum
+// of the columns of P' in bit-sliced counters (four words of sum bits; 9
+// instructions for three columns), and the best pivot falls out of them from
+// the top bit down. The columns and the frames of the first kLsRegs levels
+// are registers; a clique found is one word in LDS (the members chosen since
+// the subtree's root), hashed and counted later by full waves: with hash sums
+// carried from node to node and frames in memory, a step waited for loads
+// that missed the L2.
+//
+// Enumeration in ms, without it -> with it (donating alike): Chung-Lu 2^17
+// 21.5 -> 15.4, R-MAT 14 25 -> 21.4, R-MAT 12 5.4 -> 3.0; against subtrees of
+// at most 16 members, one 32-bit column each: R-MAT 14 29.6 -> 21.4, a batch
+// of 2.8 G nodes 617 -> 405 (whole call). About 29 of the 64 lanes are busy in
+// a step; the rest have run out of work in their subtree.
+//
+// Members keep their order (S indices, then outside rows) within P and
+// within X; byte r of `xb` says how many X members come before P member r,
+// which decides a tie between the two. Pivots (largest |P & N(u)|, ties to
+// the lowest member) and child order are those of the small-universe solver,
+// so the same nodes are visited.
+constexpr uint32_t kLsP = 15, kLsX = 48, kLsSlots = 64;
+// A wave's region in device memory: a slot per subtree ({column words 0, 1}
+// of 16 P members, 16 bytes xb, {p | x << 8 | |R| << 16}, root, R's hash
+// sum), the hash terms of its P members, and the frames past kLsRegs levels
+// {P | X of P's members << 16, X (two words), the pivot's row | chosen members
+// << 16}, level-major. A pushed level has |P| >= 3 and each level at least
+// one member fewer than its parent's. In LDS: the cliques found and not
+// counted yet, {chosen members | slot << 16}.
+constexpr uint32_t kLsLevels = kLsP - 3, kLsRegs = 4;
+constexpr uint32_t kLsXbAt = 128, kLsHeadAt = 144, kLsSlotBytes = 160, kLsHOff = kLsSlots * kLsSlotBytes,
+                   kLsFrOff = kLsHOff + kLsSlots * 16 * 8, kLsBytes = kLsFrOff + (kLsLevels - kLsRegs) * kLsSlots * 16;
+constexpr uint32_t kLsFound = 512, kLsLds = kLsFound * 4;
 // busy lanes at which the wave takes over the rest of their subtrees
-constexpr uint32_t kLsDrain = 6;
-typedef __attribute__((address_space(3))) uint16_t lds_u16;
+constexpr uint32_t kLsDrain = 4;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
+typedef __attribute__((address_space(1))) uint8_t glb_u8;
+typedef __attribute__((address_space(1))) u32x2 glb_u32x2;
+typedef __attribute__((address_space(1))) u32x4 glb_u32x4;
 
 struct LsOut {
   uint64_t count, nodes, hash;
   uint32_t max_size;
 };
 
-// Queues the subtree of a small-universe node: K = its members (P | X) over
-// the solver's numbering, Pk = its P, rb = |R| there, mix = R's hash sum; the
-// calling lane i holds member i's row M and hash term hs. Wave-uniform call
-// with a free slot.
-template <typename Mk>
-__device__ __forceinline__ void ls_put(WaveAcc &wa, Mk M, uint64_t hs, Mk K, Mk Pk, uint32_t rb, uint64_t mix) {
-  using O = MaskOps<Mk>;
-  const uint32_t L = lane_id(), j = wa.ls_n, nk = O::popc(K);
-  const bool in = lane_in(O::lanes(K));
-  const uint32_t k = mbcnt((uint64_t)K);  // the member's new index
-  uint32_t row;
-  if ((K & (K + 1)) == 0) {
-    row = (uint32_t)(M & K);  // members 0..k-1 keep their numbers
-  } else {
-    row = 0;
-    uint32_t t = 0;
-    for (Mk kk = K; kk; kk &= kk - 1, ++t) row |= (uint32_t)((M >> O::ctz(kk)) & 1u) << t;
-  }
-  lds_u16 *rows = (lds_u16 *)(uintptr_t)wa.ls_lds;
-  if (in) {
-    rows[j * kLsMax + k] = (uint16_t)row;
-    wa.ls_h[j * kLsMax + k] = hs;
-  }
-  // P over the new indices: every member's P flag moves to lane k
-  const uint32_t f = (uint32_t)__builtin_amdgcn_ds_permute((int)((in ? k : kWave - 1) * 4),
-                                                           lane_in(O::lanes(Pk)) ? 1 : 0);
-  const uint32_t pk = (uint32_t)ballot(L < nk && f != 0);
-  if (L == 0) {
-    u32x4 *hdr = (u32x4 *)((uint8_t *)wa.ls_h + kLsHdrOff);
-    hdr[j] = u32x4{pk | nk << 16, rb, (uint32_t)mix, (uint32_t)(mix >> 32)};
-  }
-  wa.ls_n = j + 1;
-  wa.ls_u = max(wa.ls_u, nk);
+__device__ __forceinline__ bool ls_fits(const BkParams &pr, uint32_t p, uint32_t x) {
+  return p + x <= pr.ls_max && p <= kLsP && x <= kLsX;
 }
 
-// Pivot of a lane's node: the member u of P | X with the most members of P
-// among its neighbours, ties to the lowest u. False when that count is |P|
-// (no child). R: the lane's 16 rows; um: members to scan (uniform).
-__device__ __forceinline__ bool ls_pick(const lds_u16 *R, uint32_t P, uint32_t X, uint32_t um, uint32_t &piv) {
-  const u32x4 w0 = *(const lds_u32x4 *)R;
-  u32x4 w1 = {0, 0, 0, 0};
-  if (um > 8) w1 = *(const lds_u32x4 *)(R + 8);
-  const uint32_t PX = P | X, Ph = P << 16;
-  uint32_t best = 0;
-#pragma unroll
-  for (uint32_t u = 0; u < kLsMax; ++u) {
-    if (u >= um) break;
-    const uint32_t w = u < 8 ? w0[u >> 1] : w1[(u - 8) >> 1];
-    // key: count << 5 | (31 - u), so the maximum picks the lowest u of the best count
-    const uint32_t c = (uint32_t)__builtin_popcount(w & ((u & 1) ? Ph : P));
-    const uint32_t key = (c << 5) | (31u - u);
-    best = max(best, ((PX >> u) & 1u) ? key : 0u);
+// Queues a subtree of p members of P and x of X (a free slot is the caller's).
+// Lane r < p holds the column of P member r (c0, c1), its hash term and the
+// number of X members before it; rb = |R|, mix = R's hash sum.
+__device__ __forceinline__ void ls_put(WaveAcc &wa, uint32_t p, uint32_t x, uint32_t c0, uint32_t c1, uint64_t hs,
+                                       uint32_t xb, uint32_t rb, uint32_t root, uint64_t mix) {
+  const uint32_t j = wa.ls_n, L = lane_id();
+  uint8_t *slot = wa.ls + j * kLsSlotBytes;
+  if (L < p) {
+    ((glb_u32x2 *)slot)[L] = u32x2{c0, c1};
+    ((glb_u8 *)(slot + kLsXbAt))[L] = (uint8_t)xb;
+    ((glb_u64 *)(wa.ls + kLsHOff))[j * 16 + L] = hs;
   }
-  piv = 31u - (best & 31u);
-  return best != 0 && (best >> 5) != (uint32_t)__builtin_popcount(P);
+  if (L == 0) *(glb_u32x4 *)(slot + kLsHeadAt) = u32x4{p | x << 8 | rb << 16, root, (uint32_t)mix, (uint32_t)(mix >> 32)};
+  wa.ls_n = j + 1;
+  wa.ls_p = max(wa.ls_p, p);
+  wa.ls_x = max(wa.ls_x, x);
 }
 
 // The small-universe solver's loop over a renumbered universe: lane i holds
 // member i's row M over the members and its hash term hs; lP / lX are the
-// root's P and X over the members.
-template <typename Mk, int kStat>
+// root's P and X over the members. Of a member that is in X from the start
+// only the row's bits of P's members are used. kResume: the root is a node
+// whose pivot row Np0 is known (its remaining children are solved).
+template <int kStat>
+__device__ __forceinline__ void ls_flush(const BkParams &pr, lds_ull *hist_lds, WaveAcc &wa);
+
+template <typename Mk, int kStat, bool kResume = false>
 __device__ __forceinline__ void small_loop(const BkParams &pr, Mk M, uint64_t hs, Mk lP, Mk lX, uint64_t mix,
-                                           uint32_t rbase, unsigned long long *hist_lds, WaveAcc &wa,
-                                           Clock<kStat> &clk, int piv0 = -1) {
+                                           uint32_t rbase, uint32_t root, lds_ull *hist_lds, WaveAcc &wa,
+                                           Clock<kStat> &clk, Mk Np0 = 0) {
   using O = MaskOps<Mk>;
   // pivot over P | X (the lowest member among the best scores): false when
   // it covers P (no child)
@@ -1606,15 +1757,16 @@ __device__ __forceinline__ void small_loop(const BkParams &pr, Mk M, uint64_t hs
     return mx != 0 && mx - 1u != O::popc(P);
   };
   clk.to(kBdPivot);
-  Mk P = lP, X = lX;
-  uint32_t piv;
-  if (piv0 >= 0) piv = (uint32_t)piv0;  // a node whose pivot is known: its remaining children
-  else if (!pick(P, X, piv)) return;
-  Mk Np = O::rd(M, piv);
+  Mk P = lP, X = lX, Np = Np0;
+  if constexpr (!kResume) {
+    uint32_t piv;
+    if (!pick(P, X, piv)) return;
+    Np = O::rd(M, piv);
+  }
   uint32_t d = 0;
   // frames: lane d of each register holds level d
-  Mk fP = 0, fX = 0;
-  uint32_t fV = 0, fMl = 0, fMh = 0;
+  Mk fP = 0, fX = 0, fN = 0;
+  uint32_t fMl = 0, fMh = 0;
   // tallies of this subtree, added to the wave's totals at the end; the
   // cliques' hash terms and histogram bins are taken 64 at a time
   WaveAcc t{};
@@ -1632,8 +1784,7 @@ __device__ __forceinline__ void small_loop(const BkParams &pr, Mk M, uint64_t hs
       P = O::rd(fP, d);
       X = O::rd(fX, d);
       mix = ((uint64_t)rdlane(fMh, d) << 32) | rdlane(fMl, d);
-      piv = rdlane(fV, d);
-      Np = O::rd(M, piv);
+      Np = O::rd(fN, d);
       continue;
     }
     const Mk cb = B & (~B + 1);
@@ -1687,10 +1838,28 @@ __device__ __forceinline__ void small_loop(const BkParams &pr, Mk M, uint64_t hs
       if ((Xn & (piv_a ? Mb : Ma)) == 0) keep_clique(pr, hist_lds, t, kb, rbase + d + 2, cmix + (piv_a ? hb : ha));
       continue;
     }
-    if (lane_of(kStat) && O::popc(Pn | Xn) <= pr.ls_max && wa.ls_n < kLsSlots) {
-      clk.to(kBdBranch);
-      ls_put<Mk>(wa, M, hs, Pn | Xn, Pn, rbase + d + 1, cmix);
-      continue;
+    if constexpr (lane_of(kStat)) {
+      if (ls_fits(pr, np, O::popc(Xn))) {
+        if (wa.ls_n == kLsSlots) ls_flush<kStat>(pr, hist_lds, wa);
+        // members move to their lanes in a queued subtree, P's to 0.., X's to
+        // 16.. (all others to lane 15, which no member has)
+        const uint64_t mP = O::lanes(Pn), mX = O::lanes(Xn);
+        const bool inP = lane_in(mP), inX = lane_in(mX);
+        const uint32_t r = mbcnt(mP), x = mbcnt(mX), dst = 4 * (inP ? r : inX ? 16 + x : 15u);
+        const Mk Mq = O::permute(dst, M);
+        const uint64_t hq = MaskOps<uint64_t>::permute(dst, hs);
+        const uint32_t xbq = (uint32_t)__builtin_amdgcn_ds_permute((int)dst, (int)x);
+        const uint32_t nx = O::popc(Xn), L = lane_id();
+        const bool on = L < np || (L >= 16 && L < 16 + nx);
+        uint32_t c0 = 0, c1 = 0, k = 0;
+        for (Mk m = Pn; m; m &= m - 1, ++k) {
+          const uint64_t col = ballot(on && ((Mq >> O::ctz(m)) & 1u));
+          c0 = wrlane(c0, k, (uint32_t)col);
+          c1 = wrlane(c1, k, (uint32_t)(col >> 32));
+        }
+        ls_put(wa, np, nx, c0, c1, hq, xbq, rbase + d + 1, root, cmix);
+        continue;
+      }
     }
     clk.to(kBdPivot);
     uint32_t npiv;
@@ -1700,13 +1869,12 @@ __device__ __forceinline__ void small_loop(const BkParams &pr, Mk M, uint64_t hs
     fX = O::wr(fX, d, X);
     fMl = wrlane(fMl, d, (uint32_t)mix);
     fMh = wrlane(fMh, d, (uint32_t)(mix >> 32));
-    fV = wrlane(fV, d, piv);
+    fN = O::wr(fN, d, Np);
     ++d;
     P = Pn;
     X = Xn;
     mix = cmix;
-    piv = npiv;
-    Np = O::rd(M, piv);
+    Np = O::rd(M, npiv);
   }
   if (kb.n) flush_cliques(pr, hist_lds, kb);
   wa.nodes += t.nodes;
@@ -1716,131 +1884,259 @@ __device__ __forceinline__ void small_loop(const BkParams &pr, Mk M, uint64_t hs
   wa.max_size = max(wa.max_size, t.max_size);
 }
 
-// Runs the n queued subtrees, lane j the subtree of slot j, node for node as
-// the small-universe solver would (the |P| <= 2 shortcuts included). um: the
-// largest member count among them. Once at most kLsDrain lanes are still
-// busy, the wave takes over: each such lane's remaining work (the open
-// children of its current node and of every frame below it) runs through
-// the small-universe solver's loop, which resumes a node at its known pivot,
-// so one large subtree does not hold the other lanes idle. Returns the
-// totals.
-__device__ __noinline__ LsOut ls_run(uint32_t n, uint32_t um, uint32_t lds, const uint64_t *hg, uint32_t hist_lds_addr,
-                                     uint32_t hist_lds_n, unsigned long long *hist, uint32_t hist_len) {
+// A word of the 16 picked by a lane's index. (Vectors, not arrays: an array
+// indexed so goes to memory.)
+__device__ __forceinline__ uint32_t ls_pick16(u32x16 w, uint32_t i) {
+  const u32x8 a = (i & 8u) ? w.hi : w.lo;
+  const u32x4 b = (i & 4u) ? a.hi : a.lo;
+  const uint32_t c0 = (i & 2u) ? b[2] : b[0], c1 = (i & 2u) ? b[3] : b[1];
+  return (i & 1u) ? c1 : c0;
+}
+
+// Does P member r come after X member x in the members' order (xb)?
+__device__ __forceinline__ bool ls_after(u32x4 xb, uint32_t r, uint32_t x) {
+  const uint32_t t01 = (r & 4u) ? xb[1] : xb[0], t23 = (r & 4u) ? xb[3] : xb[2];
+  return ((((r & 8u) ? t23 : t01) >> (8 * (r & 3u))) & 0xFFu) > x;
+}
+
+// Bit-sliced counters: bit u of s[3..0] is the count of member u, at most 15.
+struct LsCount {
+  uint32_t s0 = 0, s1 = 0, s2 = 0, s3 = 0;
+  // adds three words
+  __device__ __forceinline__ void add3(uint32_t a, uint32_t b, uint32_t c) {
+    const uint32_t x = a ^ b ^ c, y = (a & b) | (c & (a ^ b));
+    const uint32_t c0 = s0 & x;
+    s0 ^= x;
+    const uint32_t z = (y & c0) | (s1 & (y ^ c0));
+    s1 ^= y ^ c0;
+    const uint32_t c2 = s2 & z;
+    s2 ^= z;
+    s3 |= c2;
+  }
+};
+
+// Runs the n queued subtrees, lane j the subtree of slot j. A step takes one
+// child of a lane's node (after one pop, if its node has none left) and
+// decides it: leaf, at most two vertices left (decided without a child, as in
+// the wave-wide loop), covered, or a new node. maxp / maxx: the most members
+// of P and X among the subtrees. Once at most kLsDrain lanes are still busy,
+// the wave takes over: each such lane's remaining work (the open children of
+// its current node and of every frame below it) runs through the
+// small-universe solver's loop, so that one large subtree does not hold the
+// other lanes idle. Returns the totals; the subtrees' own counts go to their
+// roots' labels.
+__device__ __noinline__ __attribute__((not_tail_called)) LsOut ls_run(uint32_t n, uint32_t maxp, uint32_t maxx, uint8_t *ls, uint32_t ls_lds,
+                                     uint32_t hist_lds_addr, uint32_t hist_lds_n, unsigned long long *hist,
+                                     uint32_t hist_len, unsigned long long *sub_nodes,
+                                     unsigned long long *sub_cliques) {
   n = uniform(n);
-  um = uniform(um);
-  lds = uniform(lds);
+  maxp = uniform(maxp);
+  maxx = uniform(maxx);
+  ls_lds = uniform(ls_lds);
   hist_lds_addr = uniform(hist_lds_addr);
   hist_lds_n = uniform(hist_lds_n);
   hist_len = uniform(hist_len);
+  ls = (uint8_t *)uniform64((uint64_t)(uintptr_t)ls);
+  hist = (unsigned long long *)uniform64((uint64_t)(uintptr_t)hist);
   const uint32_t L = lane_id();
-  // the queue's device-memory writes (hash terms, headers) precede these reads
-  __builtin_amdgcn_s_waitcnt(0);
-  const lds_u16 *R = (const lds_u16 *)(uintptr_t)lds + L * kLsMax;
-  const glb_u32 *hdr = (const glb_u32 *)((const uint8_t *)hg + kLsHdrOff) + 4 * L;
-  glb_u32 *fr = (glb_u32 *)((uint8_t *)hg + kLsFrOff) + L;
-  typedef __attribute__((address_space(3))) unsigned long long lds_ull;
+  // the queue's writes precede these reads
+  drain();
   lds_ull *hist_lds = (lds_ull *)(uintptr_t)hist_lds_addr;
-  const glb_u64 *H = (const glb_u64 *)hg + L * kLsMax;
-  uint32_t cnt = 0, nodes = 0, maxs = 0;
-  uint64_t hacc = 0;
-  auto emit = [&](uint32_t size, uint64_t m) {
-    ++cnt;
-    maxs = max(maxs, size);
-    hacc += clique_hash(m, size);
-    if (size < hist_lds_n) __hip_atomic_fetch_add(&hist_lds[size], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    else atomicAdd(&hist[min(size, hist_len - 1)], 1ull);
-  };
-  uint32_t P = 0, X = 0, piv = 0, d = 0, rb = 0, Np = 0;
-  uint64_t mix = 0, path = 0, pivs = 0;
-  bool act = L < n;
-  uint32_t h0 = 0;
+  lds_u32 *found = (lds_u32 *)(uintptr_t)ls_lds;
+  const glb_u64 *H = (const glb_u64 *)(ls + kLsHOff);
+  glb_u32x4 *fr = (glb_u32x4 *)(ls + kLsFrOff) + L;
+  const bool wide = maxx > 16;  // some subtree has X members past the first word
+  u32x16 A = 0, B = 0;          // columns: words 0 and 1
+  u32x4 xb = 0;
+  // the lane's node: P and X over P's members (PX = P | X << 16), X's members
+  // (X0 << 16: the first 16 as in A; X1), the pivot's row | members chosen
+  // since the subtree's root << 16, depth
+  uint32_t PX = 0, X0 = 0, X1 = 0, NR = 0, d = 0;
+  uint32_t fP[kLsRegs], fX0[kLsRegs], fX1[kLsRegs], fN[kLsRegs];
+#pragma unroll
+  for (uint32_t k = 0; k < kLsRegs; ++k) fP[k] = fX0[k] = fX1[k] = fN[k] = 0;
+  bool act = L < n, fresh = true;  // fresh: the subtree's root, not decided yet
   if (act) {
-    h0 = hdr[0];
-    P = h0 & 0xFFFFu;
-    X = ((1u << (h0 >> 16)) - 1u) & ~P;
-    rb = hdr[1];
-    mix = (uint64_t)hdr[2] | (uint64_t)hdr[3] << 32;
-    act = ls_pick(R, P, X, um, piv);
-    if (act) Np = R[piv];
+    const glb_u32x4 *sl = (const glb_u32x4 *)(ls + L * kLsSlotBytes);
+    const uint32_t head = ((const glb_u32 *)(ls + L * kLsSlotBytes + kLsHeadAt))[0];
+    xb = sl[kLsXbAt / 16];
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
+      const u32x4 q = sl[k];
+      A[2 * k] = q[0];
+      B[2 * k] = q[1];
+      A[2 * k + 1] = q[2];
+      B[2 * k + 1] = q[3];
+    }
+    const uint32_t p = head & 0xFFu, x = (head >> 8) & 0xFFu;
+    PX = (1u << p) - 1u;
+    X0 = x < 16 ? ((1u << x) - 1u) << 16 : 0xFFFF0000u;
+    X1 = x > 16 ? 0xFFFFFFFFu >> (48u - x) : 0u;
   }
+  uint32_t cnt = 0, nodes = 0, nf = 0;  // the lane's cliques and nodes; cliques in `found`
+  LsOut o{};
+  uint64_t hacc = 0;
+  uint32_t maxs = 0;
+  // hashes and counts the cliques in `found`, one per lane
+  auto count_found = [&]() {
+    for (uint32_t b = 0; b < nf; b += kWave) {
+      if (b + L < nf) {
+        const uint32_t rec = found[b + L], j = rec >> 16;
+        const u32x4 hd = *(const glb_u32x4 *)(ls + j * kLsSlotBytes + kLsHeadAt);
+        uint64_t m = (uint64_t)hd[2] | (uint64_t)hd[3] << 32;
+        const uint32_t sel = rec & 0xFFFFu, size = (hd[0] >> 16) + (uint32_t)__builtin_popcount(sel);
+        for (uint32_t q = sel; q; q &= q - 1) m += H[j * 16 + (uint32_t)__builtin_ctz(q)];
+        hacc += clique_hash(m, size);
+        maxs = max(maxs, size);
+        if (size < hist_lds_n) __hip_atomic_fetch_add(&hist_lds[size], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        else atomicAdd(&hist[min(size, hist_len - 1)], 1ull);
+      }
+    }
+    nf = 0;
+  };
   while (true) {
     if (popc64(ballot(act)) <= kLsDrain) break;
-    if (!act) continue;
-    const uint32_t B = P & ~Np;
-    if (B == 0) {
-      if (d == 0) {
-        act = false;
-        continue;
-      }
-      --d;
-      const uint32_t f = fr[d * kLsSlots], sh = 4 * d;
-      P = f & 0xFFFFu;
-      X = f >> 16;
-      mix -= H[(uint32_t)(path >> sh) & 15u];
-      piv = (uint32_t)(pivs >> sh) & 15u;
-      Np = R[piv];
-      continue;
-    }
-    const uint32_t c = (uint32_t)__builtin_ctz(B), cb = 1u << c;
-    P ^= cb;
-    X |= cb;
-    const uint32_t Mc = R[c];
-    const uint32_t Pn = P & Mc, Xn = X & Mc;
-    ++nodes;
-    const uint64_t cmix = mix + H[c];
-    if (Pn == 0) {
-      if (Xn == 0) emit(rb + d + 1, cmix);
-      continue;
-    }
-    const uint32_t np = (uint32_t)__builtin_popcount(Pn);
-    if (np <= 2) {
-      const uint32_t a = (uint32_t)__builtin_ctz(Pn), Ma = R[a];
-      const uint64_t ha = H[a];
-      if (np == 1) {
-        if ((Xn & Ma) == 0) {
-          ++nodes;
-          emit(rb + d + 2, cmix + ha);
+    if (nf > kLsFound - 2 * kWave) count_found();  // a step finds at most two cliques a lane
+    uint32_t e1 = 0, e2 = 0;  // members of the cliques the lane finds
+    if (act) {
+      // pop one level if the node has no child left
+      uint32_t ch = PX & ~NR & 0xFFFFu;
+      if (ch == 0 && !fresh) {
+        act = d != 0;
+        if (act) {
+          --d;
+          if (d >= kLsRegs) {
+            const u32x4 f = fr[(d - kLsRegs) * kLsSlots];
+            PX = f[0];
+            X0 = f[1];
+            X1 = f[2];
+            NR = f[3];
+          } else {
+#pragma unroll
+            for (uint32_t k = 0; k < kLsRegs; ++k) {
+              PX = d == k ? fP[k] : PX;
+              X0 = d == k ? fX0[k] : X0;
+              X1 = d == k ? fX1[k] : X1;
+              NR = d == k ? fN[k] : NR;
+            }
+          }
+          ch = PX & ~NR & 0xFFFFu;
         }
-        continue;
       }
-      const uint32_t b = (uint32_t)__builtin_ctz(Pn & (Pn - 1)), Mb = R[b];
-      const uint64_t hb = H[b];
-      if (Xn & Ma & Mb) continue;  // an X member covers P
-      if ((Ma >> b) & 1u) {
-        nodes += 2;
-        emit(rb + d + 3, cmix + ha + hb);
-        continue;
+      // the node to decide: a child of the lane's node, or the root itself
+      const bool go = fresh || ch != 0;
+      const uint32_t c = fresh || !go ? 0u : (uint32_t)__builtin_ctz(ch);
+      const uint32_t ca = fresh ? ~0u : ls_pick16(A, c);
+      if (go && !fresh) {
+        PX ^= 0x10001u << c;  // c leaves P for X
+        ++nodes;
       }
-      const uint32_t xs = Xn & (Ma | Mb);
-      if (xs == 0) {
-        nodes += 2;
-        emit(rb + d + 2, cmix + ha);
-        emit(rb + d + 2, cmix + hb);
-        continue;
+      const uint32_t sel = fresh ? 0u : (NR >> 16) | 1u << c;
+      const uint32_t Pn = PX & ca & 0xFFFFu, Qn = (PX >> 16) & ca, Xa = X0 & ca;
+      const uint32_t Ca = Pn | Qn | Xa;  // pivot candidates
+      uint32_t Cb = 0;
+      if (wide) Cb = X1 & (fresh ? ~0u : ls_pick16(B, c));
+      // scores of all members: the sum of the columns of P'
+      LsCount sa, sb;
+      auto col = [&](u32x16 w, uint32_t r) -> uint32_t {
+        return w[r] & (uint32_t)__builtin_amdgcn_sbfe((int)Pn, r, 1);
+      };
+#pragma unroll
+      for (uint32_t r = 0; r < kLsP; r += 3)
+        if (r == 0 || r < maxp) {
+          sa.add3(col(A, r), col(A, r + 1), col(A, r + 2));
+          if (wide) sb.add3(col(B, r), col(B, r + 1), col(B, r + 2));
+        }
+      // the candidates with the best score, from its top bit down
+      uint32_t Ka = Ca, Kb = Cb, best = 0;
+      auto top = [&](uint32_t pa, uint32_t pb, uint32_t bit) {
+        const uint32_t ta = Ka & pa, tb = wide ? Kb & pb : 0u;
+        const bool any = (ta | tb) != 0;
+        Ka = any ? ta : Ka;
+        if (wide) Kb = any ? tb : Kb;
+        best |= any ? bit : 0u;
+      };
+      top(sa.s3, sb.s3, 8);
+      top(sa.s2, sb.s2, 4);
+      top(sa.s1, sb.s1, 2);
+      top(sa.s0, sb.s0, 1);
+      // the pivot: the lowest of them in the members' order (xb)
+      const uint32_t kp = Ka & 0xFFFFu, kx = Ka >> 16;
+      const uint32_t pr = kp ? (uint32_t)__builtin_ctz(kp) : 0u;
+      const uint32_t px = kx ? (uint32_t)__builtin_ctz(kx) : 16u + (Kb ? (uint32_t)__builtin_ctz(Kb) : 0u);
+      const bool isx = kp == 0 || ((kx | Kb) != 0 && ls_after(xb, pr, px));
+      // its row: its bit of every column
+      const uint32_t at = isx ? px + 16u : pr;
+      uint32_t piv = 0;
+#pragma unroll
+      for (uint32_t r = 0; r < kLsP; r += 3)
+        if (r == 0 || r < maxp) {
+#pragma unroll
+          for (uint32_t k = r; k < r + 3; ++k) {
+            const uint32_t w = wide && at >= 32 ? B[k] : A[k];
+            piv |= ((w >> (at & 31u)) & 1u) << k;
+          }
+        }
+      const uint32_t np = (uint32_t)__builtin_popcount(Pn);
+      if (go && np >= 3 && best < np) {
+        // a node of its own
+        if (!fresh) {
+          if (d >= kLsRegs) {
+            fr[(d - kLsRegs) * kLsSlots] = u32x4{PX, X0, X1, NR};
+          } else {
+#pragma unroll
+            for (uint32_t k = 0; k < kLsRegs; ++k) {
+              fP[k] = d == k ? PX : fP[k];
+              fX0[k] = d == k ? X0 : fX0[k];
+              fX1[k] = d == k ? X1 : fX1[k];
+              fN[k] = d == k ? NR : fN[k];
+            }
+          }
+          ++d;
+        }
+        PX = Pn | Qn << 16;
+        X0 = Xa;
+        X1 = Cb;
+        NR = piv | sel << 16;
+        fresh = false;
+      } else if (go) {
+        act = !fresh;  // a root decided here has no node of its own
+        if (np == 0) {
+          e1 = (Ca | Cb) == 0 ? sel : 0u;
+        } else if (np == 1) {
+          nodes += best == 0;
+          e1 = best == 0 ? sel | Pn : 0u;
+        } else if (np == 2 && best < 2) {  // at 2 an X member covers P
+          const uint32_t a = (uint32_t)__builtin_ctz(Pn), b = 31u - (uint32_t)__builtin_clz(Pn);
+          if ((sa.s0 >> a) & 1u) {  // a sees b
+            nodes += 2;
+            e1 = sel | Pn;
+          } else if (best == 0) {
+            nodes += 2;
+            e1 = sel | 1u << a;
+            e2 = sel | 1u << b;
+          } else {
+            // the pivot is an X member adjacent to one of a, b (a and b see
+            // neither); the child is the other, maximal if no X member sees it
+            const uint32_t o1 = (piv >> a) & 1u ? b : a;
+            ++nodes;
+            uint32_t cov = Ca & ls_pick16(A, o1);
+            if (wide) cov |= Cb & ls_pick16(B, o1);
+            e1 = cov == 0 ? sel | 1u << o1 : 0u;
+          }
+        }
       }
-      // the pivot is the lowest X member adjacent to one of a, b; the child
-      // is the other one
-      const bool piv_a = (Ma >> __builtin_ctz(xs)) & 1u;
-      ++nodes;
-      if ((Xn & (piv_a ? Mb : Ma)) == 0) emit(rb + d + 2, cmix + (piv_a ? hb : ha));
-      continue;
     }
-    uint32_t npiv;
-    if (!ls_pick(R, Pn, Xn, um, npiv)) continue;
-    fr[d * kLsSlots] = P | X << 16;
-    const uint32_t sh = 4 * d;
-    path = (path & ~(15ull << sh)) | (uint64_t)c << sh;
-    pivs = (pivs & ~(15ull << sh)) | (uint64_t)piv << sh;
-    ++d;
-    P = Pn;
-    X = Xn;
-    mix = cmix;
-    piv = npiv;
-    Np = R[piv];
+    const uint64_t m1 = ballot(e1 != 0), m2 = ballot(e2 != 0);
+    if (e1) found[nf + mbcnt(m1)] = e1 | L << 16;
+    nf += popc64(m1);
+    if (m2) {
+      if (e2) found[nf + mbcnt(m2)] = e2 | L << 16;
+      nf += popc64(m2);
+    }
+    cnt += (e1 != 0) + (e2 != 0);
   }
-  LsOut o;
-  o.count = wave_sum(cnt);
-  o.nodes = wave_sum(nodes);
+  count_found();
   o.hash = wave_add64(hacc);
   o.max_size = wave_max(maxs);
   // the busy lanes' remaining work, on the whole wave
@@ -1848,272 +2144,359 @@ __device__ __noinline__ LsOut ls_run(uint32_t n, uint32_t um, uint32_t lds, cons
   q.hist = hist;
   q.hist_len = hist_len;
   q.hist_lds = hist_lds_n;
-  WaveAcc w{};
   Clock<kStatNone> clk;
-  const lds_u16 *rows = (const lds_u16 *)(uintptr_t)lds;
-  const glb_u32 *frs = (const glb_u32 *)((const uint8_t *)hg + kLsFrOff);
   for (uint64_t left = ballot(act); left; left &= left - 1) {
     const uint32_t j = ctz64(left);
-    // slot j's rows and hash terms, member k on lane k
-    const uint32_t nm = rdlane(h0, j) >> 16;
-    const uint32_t M = L < nm ? rows[j * kLsMax + L] : 0u;
-    const uint64_t hs = L < nm ? ((const glb_u64 *)hg)[j * kLsMax + L] : 0ull;
-    uint32_t Pk = rdlane(P, j), Xk = rdlane(X, j), pk = rdlane(piv, j);
-    uint64_t mk = rdlane64(mix, j);
-    const uint32_t dj = rdlane(d, j), rbj = rdlane(rb, j);
-    const uint64_t pathj = rdlane64(path, j), pivsj = rdlane64(pivs, j);
+    // the members of slot j in their order, one per lane: P member r at
+    // position r + xb[r]
+    const uint8_t *slot = ls + j * kLsSlotBytes;
+    const u32x4 hd = *(const glb_u32x4 *)(slot + kLsHeadAt);
+    const uint32_t h0 = uniform(hd[0]);
+    const uint32_t p = h0 & 0xFFu, nm = p + ((h0 >> 8) & 0xFFu), rbj = h0 >> 16;
+    const uint64_t mixj = uniform64((uint64_t)hd[2] | (uint64_t)hd[3] << 32);
+    const uint32_t pos = L < p ? L + ((const glb_u8 *)(slot + kLsXbAt))[L] : 0u;
+    const u32x2 cw = L < p ? ((const glb_u32x2 *)slot)[L] : u32x2{0u, 0u};
+    uint64_t mP = 0;
+    for (uint32_t r = 0; r < p; ++r) mP |= 1ull << rdlane(pos, r);
+    const uint32_t r = mbcnt(mP);
+    const bool inP = lane_in(mP), in = L < nm;
+    const uint32_t ix = inP ? r : 16u + (L - r);  // the lane's member's bit in a column
+    const uint64_t hs = inP ? H[j * 16 + r] : 0ull;
+    // rows over the members: a P member's is its column, of an X member only
+    // the bits of P's members
+    uint64_t M = 0;
+    for (uint32_t k = 0; k < p; ++k) {
+      const uint32_t to = rdlane(pos, k);
+      const uint64_t ck = (uint64_t)rdlane(cw[1], k) << 32 | rdlane(cw[0], k);
+      const bool t = in && ((ck >> (ix & 63u)) & 1ull);
+      const uint64_t cb = ballot(t);
+      if (L == to) M = cb;
+      else if (!inP && t) M |= 1ull << to;
+    }
+    WaveAcc t{};
+    uint32_t PXk = rdlane(PX, j), X0k = rdlane(X0, j), X1k = rdlane(X1, j), Nk = rdlane(NR, j);
+    const uint32_t dj = rdlane(d, j);
+    const bool fj = (ballot(fresh) >> j) & 1ull;
     for (uint32_t k = dj + 1; k-- > 0;) {
       if (k < dj) {
-        const uint32_t f = frs[k * kLsSlots + j], sh = 4 * k;
-        Pk = f & 0xFFFFu;
-        Xk = f >> 16;
-        mk -= rdlane64(hs, (uint32_t)(pathj >> sh) & 15u);
-        pk = (uint32_t)(pivsj >> sh) & 15u;
+        if (k >= kLsRegs) {
+          const u32x4 f = ((const glb_u32x4 *)(ls + kLsFrOff))[(k - kLsRegs) * kLsSlots + j];
+          PXk = uniform(f[0]);
+          X0k = uniform(f[1]);
+          X1k = uniform(f[2]);
+          Nk = uniform(f[3]);
+        } else {
+#pragma unroll
+          for (uint32_t i = 0; i < kLsRegs; ++i)
+            if (i == k) {
+              PXk = rdlane(fP[i], j);
+              X0k = rdlane(fX0[i], j);
+              X1k = rdlane(fX1[i], j);
+              Nk = rdlane(fN[i], j);
+            }
+        }
       }
-      small_loop<uint32_t, kStatNone>(q, M, hs, Pk, Xk, mk, rbj + k, (unsigned long long *)hist_lds, w, clk,
-                                      (int)pk);
+      // the node's sets over the members; R: the slot's R and those chosen since
+      const uint64_t xk = (uint64_t)X1k << 32 | X0k;
+      const uint64_t Pk = ballot(inP && ((PXk >> r) & 1u));
+      const uint64_t Qk = ballot(in && (inP ? (PXk >> (16 + r)) & 1u : (uint32_t)(xk >> (ix & 63u)) & 1u));
+      const uint64_t Nm = ballot(inP && ((Nk >> r) & 1u));
+      uint64_t mk = mixj;
+      for (uint64_t m = ballot(inP && ((Nk >> (16 + r)) & 1u)); m; m &= m - 1) mk += rdlane64(hs, ctz64(m));
+      if (fj)
+        small_loop<uint64_t, kStatNone>(q, M, hs, Pk, Qk, mk, rbj, 0, hist_lds, t, clk);
+      else
+        small_loop<uint64_t, kStatNone, true>(q, M, hs, Pk, Qk, mk, rbj + k, 0, hist_lds, t, clk,
+                                              Nm);
     }
+    if (L == j) {
+      cnt += (uint32_t)t.count;
+      nodes += (uint32_t)t.nodes;
+    }
+    o.hash += t.hash;
+    o.max_size = max(o.max_size, t.max_size);
   }
-  o.count += w.count;
-  o.nodes += w.nodes;
-  o.hash += w.hash;
-  o.max_size = max(o.max_size, w.max_size);
+  // per-root labels: one update when the whole run belongs to one root
+  const uint32_t ncnt = wave_sum(cnt), nnodes = wave_sum(nodes);
+  if (sub_nodes || sub_cliques) {
+    const uint32_t root = L < n ? ((const glb_u32 *)(ls + L * kLsSlotBytes + kLsHeadAt))[1] : 0u, r0 = uniform(root);
+    const bool one = ballot(L < n && root != r0) == 0;
+    const bool on = one ? L == 0 : L < n;
+    if (on && sub_nodes) atomicAdd(&sub_nodes[root], (unsigned long long)(one ? nnodes : nodes));
+    if (on && sub_cliques) atomicAdd(&sub_cliques[root], (unsigned long long)(one ? ncnt : cnt));
+  }
+  o.count = ncnt;
+  o.nodes = nnodes;
   return o;
 }
 
 // Runs the wave's queue, if any, and adds its totals to the wave's.
-__device__ __forceinline__ void ls_flush(const BkParams &pr, unsigned long long *hist_lds, WaveAcc &wa) {
-  if (wa.ls_n == 0) return;
-  const LsOut o = ls_run(wa.ls_n, wa.ls_u, wa.ls_lds, wa.ls_h, (uint32_t)(uintptr_t)hist_lds, pr.hist_lds, pr.hist,
-                         pr.hist_len);
-  wa.count += o.count;
-  wa.sub_cliques += o.count;
-  wa.nodes += o.nodes;
-  wa.hash += o.hash;
-  wa.max_size = max(wa.max_size, o.max_size);
-  wa.ls_n = 0;
-  wa.ls_u = 0;
+template <int kStat>
+__device__ __forceinline__ void ls_flush(const BkParams &pr, lds_ull *hist_lds, WaveAcc &wa) {
+  if constexpr (lane_of(kStat)) {
+    if (wa.ls_n == 0) return;
+    const LsOut o = ls_run(wa.ls_n, wa.ls_p, wa.ls_x, wa.ls, wa.ls_lds, (uint32_t)(uintptr_t)hist_lds, pr.hist_lds, pr.hist,
+                           pr.hist_len, pr.sub_nodes, pr.sub_cliques);
+    // (the results of a call are uniform, but only this says so)
+    wa.ls_count += uniform64(o.count);
+    wa.ls_nodes += uniform64(o.nodes);
+    wa.hash += uniform64(o.hash);
+    wa.max_size = max(wa.max_size, uniform(o.max_size));
+    wa.ls_n = wa.ls_p = wa.ls_x = 0;
+  }
 }
 
+// Solves the subtree of a node whose P, X and outside rows E number at most
+// 64: numbers the members, one per lane, and queues the subtree for the lane
+// solver or works it off in the wave-wide loop.
 template <bool kWL, int kStat, bool kLA, bool kLX>
 __device__ __forceinline__ void solve_small(const BkParams &pr, const Sub &s, uint64_t Pw, uint64_t Xw, uint64_t Ew,
-                                            uint64_t mix, uint32_t rbase, unsigned long long *hist_lds, WaveAcc &wa,
+                                            uint32_t p, uint32_t x, uint64_t mix, uint32_t rbase, lds_ull *hist_lds, WaveAcc &wa,
                                             Clock<kStat> &clk) {
-  if (lane_of(kStat) && wa.ls_n > kLsSlots - kLsReserve) {
-    clk.to(kBdSetOps);
-    ls_flush(pr, hist_lds, wa);
-  }
   const uint32_t L = lane_id(), W = s.W;
   clk.to(kBdInduced);
+  const uint64_t Cw = Pw | Xw;
+  // a lane's word k of its member's row over S (mem: the member's code)
+  auto row_word = [&](uint32_t mem, bool valid, uint32_t k) -> uint64_t {
+    const uint64_t at = (uint64_t)(mem & 8191u) * W + k;
+    if (!valid) return 0;
+    return (mem & kMemOut) ? ld64<kLX>(s.XR, at) : ld64<kLA>(s.A, at);
+  };
+  if constexpr (lane_of(kStat)) {
+    // (a full queue is run from the loop below, which then meets this subtree)
+    if (wa.ls_n < kLsSlots && ls_fits(pr, p, x)) {
+      // members go to lanes, P's to 0.., X's to 16.., with the number of X
+      // members before them (each nonzero word pushes its set bits; lanes
+      // without a bit push to lane 15, which no member has)
+      uint32_t mem = 0, bp = 0, bx = 0;
+      for (uint64_t cm = ballot(Cw != 0); cm; cm &= cm - 1) {
+        const uint32_t k = ctz64(cm);
+        const uint64_t pw = rdlane64(Pw, k), xw = rdlane64(Xw, k);
+        const uint32_t rx = bx + mbcnt(xw), np = popc64(pw), nx = popc64(xw);
+        const uint32_t dst = lane_in(pw) ? bp + mbcnt(pw) : lane_in(xw) ? 16 + rx : 15u;
+        const uint32_t got = (uint32_t)__builtin_amdgcn_ds_permute((int)(dst * 4), (int)((k * 64 + L) | rx << 16));
+        if (L - bp < np || L - 16 - bx < nx) mem = got;
+        bp += np;
+        bx += nx;
+      }
+      for (uint64_t em = ballot(Ew != 0); em; em &= em - 1) {
+        const uint32_t k = ctz64(em);
+        const uint64_t w = rdlane64(Ew, k);
+        const uint32_t ne = popc64(w), dst = lane_in(w) ? 16 + bx + mbcnt(w) : 15u;
+        const uint32_t got = (uint32_t)__builtin_amdgcn_ds_permute((int)(dst * 4), (int)((k * 64 + L) | kMemOut));
+        if (L - 16 - bx < ne) mem = got;
+        bx += ne;
+      }
+      const bool on = L < p || (L >= 16 && L < 16 + x);
+      const uint64_t hs = L < p ? ld64<kLA>(s.H, mem & 8191u) : 0ull;
+      // column of P member r: the lanes whose row has its bit
+      uint32_t c0 = 0, c1 = 0, r = 0;
+      for (uint64_t pm = ballot(Pw != 0); pm; pm &= pm - 1) {
+        const uint32_t k = ctz64(pm);
+        const uint64_t pw = rdlane64(Pw, k), rw = row_word(mem, on, k);
+        for (uint32_t h = 0; h < 2; ++h) {
+          const uint32_t rh = (uint32_t)(rw >> (32 * h));
+          for (uint32_t m = (uint32_t)(pw >> (32 * h)); m; m &= m - 1, ++r) {
+            const uint64_t col = ballot((rh & m & (0u - m)) != 0);
+            c0 = wrlane(c0, r, (uint32_t)col);
+            c1 = wrlane(c1, r, (uint32_t)(col >> 32));
+          }
+        }
+      }
+      ls_put(wa, p, x, c0, c1, hs, (mem >> 16) & 0xFFu, rbase, s.root, mix);
+      return;
+    }
+  }
   // lane i <- code of member i: each nonzero word pushes its set bits to
   // consecutive lanes (lanes without a bit push to a lane outside the range)
-  const uint64_t Cw = Pw | Xw;
   uint32_t mem = 0, base = 0;
   for (uint64_t cm = ballot(Cw != 0); cm; cm &= cm - 1) {
     const uint32_t k = ctz64(cm);
     const uint64_t w = rdlane64(Cw, k), pw = rdlane64(Pw, k);
     const uint32_t cnt = popc64(w);
-    const bool in = (w >> L) & 1ull;
+    const bool in = lane_in(w);
     const uint32_t dst = in ? base + mbcnt(w) : (base + cnt) & 63u;
-    const uint32_t code = (k * 64 + L) | (((pw >> L) & 1ull) ? kMemP : 0u);
+    const uint32_t code = (k * 64 + L) | (lane_in(pw) ? kMemP : 0u);
     const uint32_t got = (uint32_t)__builtin_amdgcn_ds_permute((int)(dst * 4), (int)code);
     if (L - base < cnt) mem = got;
     base += cnt;
   }
-  const uint32_t nS = base;
   for (uint64_t em = ballot(Ew != 0); em; em &= em - 1) {
     const uint32_t k = ctz64(em);
     const uint64_t w = rdlane64(Ew, k);
     const uint32_t cnt = popc64(w);
-    const bool in = (w >> L) & 1ull;
+    const bool in = lane_in(w);
     const uint32_t dst = in ? base + mbcnt(w) : (base + cnt) & 63u;
     const uint32_t got = (uint32_t)__builtin_amdgcn_ds_permute((int)(dst * 4), (int)((k * 64 + L) | kMemOut));
     if (L - base < cnt) mem = got;
     base += cnt;
   }
   const uint32_t nm = base;
-  const bool valid = L < nm, out = (mem & kMemOut) != 0;
-  const uint32_t g = mem & 8191u;
+  const bool valid = L < nm;
   const uint64_t lP = ballot(valid && (mem & kMemP)), lX = ballot(valid && !(mem & kMemP));
-  // rows over the S members: bit j of word k's members, in member order
-  uint32_t mlo = 0, mhi = 0, j = 0;
-  for (uint64_t cm = ballot(Cw != 0); cm; cm &= cm - 1) {
-    const uint32_t k = ctz64(cm);
-    const uint64_t w = rdlane64(Cw, k);
-    uint64_t rw = 0;
-    if (valid) rw = out ? ld64<kLX>(s.XR, (uint64_t)g * W + k) : ld64<kLA>(s.A, (uint64_t)g * W + k);
+  const uint64_t hs = lane_in(lP) ? ld64<kLA>(s.H, mem & 8191u) : 0ull;
+  // rows over the members: only the bits of P's members are looked up; a P
+  // member's own row over all members is its column of them
+  uint64_t M = 0, left = lP;
+  for (uint64_t pm = ballot(Pw != 0); pm; pm &= pm - 1) {
+    const uint32_t k = ctz64(pm);
+    const uint64_t pw = rdlane64(Pw, k), rw = row_word(mem, valid, k);
     for (uint32_t h = 0; h < 2; ++h) {
-      const uint32_t r = (uint32_t)(rw >> (32 * h));
-      for (uint32_t wh = (uint32_t)(w >> (32 * h)); wh; wh &= wh - 1) {
-        const uint32_t t = (r >> __builtin_ctz(wh)) & 1u;
-        if (j < 32) mlo |= t << j;
-        else mhi |= t << (j - 32);
-        ++j;
+      const uint32_t rh = (uint32_t)(rw >> (32 * h));
+      for (uint32_t m = (uint32_t)(pw >> (32 * h)); m; m &= m - 1, left &= left - 1) {
+        const uint32_t at = uniform(ctz64(left));
+        const uint32_t t = (rh >> __builtin_ctz(m)) & 1u;
+        const uint64_t col = ballot(t != 0);
+        M |= lane_in(lP) ? 0ull : (uint64_t)t << at;
+        M = wrlane64(M, at, col);
       }
     }
   }
-  uint64_t M = ((uint64_t)mhi << 32) | mlo;
-  // S members' bits for the outside rows: the transpose of the outside rows'
-  // S bits
-  for (uint32_t e = nS; e < nm; ++e) {
-    const uint64_t re = rdlane64(M, e);
-    M |= (L < nS ? (re >> L) & 1ull : 0ull) << e;
-  }
-  const uint64_t hs = valid && !out ? ld64<kLA>(s.H, g) : 0ull;
-
-  if (lane_of(kStat) && nm <= pr.ls_max) {
-    clk.to(kBdBranch);
-    ls_put<uint32_t>(wa, (uint32_t)M, hs, (1u << nm) - 1u, (uint32_t)lP, rbase, mix);
-    return;
-  }
-  if (nm <= 32)
-    small_loop<uint32_t, kStat>(pr, (uint32_t)M, hs, (uint32_t)lP, (uint32_t)lX, mix, rbase, hist_lds, wa, clk);
+  // (the lane-solver instances keep one copy of the loop: most of what it
+  // would solve with 32-bit masks is queued)
+  if (!lane_of(kStat) && nm <= 32)
+    small_loop<uint32_t, kStat>(pr, (uint32_t)M, hs, (uint32_t)lP, (uint32_t)lX, mix, rbase, s.root, hist_lds, wa, clk);
   else
-    small_loop<uint64_t, kStat>(pr, M, hs, lP, lX, mix, rbase, hist_lds, wa, clk);
+    small_loop<uint64_t, kStat>(pr, M, hs, lP, lX, mix, rbase, s.root, hist_lds, wa, clk);
 }
 
 // Runs BK from (P, X, E) on an arena that build_bits (or a received task)
 // has filled; kLA / kLX: S and A / the outside rows are in LDS.
 template <bool kWL, int kStat, bool kLA, bool kLX>
-__device__ __forceinline__ void solve_bits_t(const BkParams &pr, Sub &s, uint64_t cP, uint64_t cX, uint64_t cE,
-                                             unsigned long long *hist_lds, WaveAcc &wa, Clock<kStat> &clk) {
+__device__ __forceinline__ void solve_bits_t(const BkParams &pr, const Sub &s, uint64_t cP, uint64_t cX, uint64_t cE,
+                                             lds_ull *hist_lds, WaveAcc &wa, Clock<kStat> &clk) {
   const uint32_t L = lane_id(), W = s.W, WX = s.WX;
   const bool act = L < W;
-  if (small_ok<kWL>(pr, cP, cX, cE)) {
-    solve_small<kWL, kStat, kLA, kLX>(pr, s, cP, cX, cE, s.rmix, s.rsize, hist_lds, wa, clk);
-    return;
-  }
-  uint32_t piv, best;
-  clk.to(kBdPivot);
-  pick_pivot_bits<kLA, kLX>(s, cP, cX, cE, piv, best);
-  if (piv == kNone || best == wave_sum(popc64(cP))) return;
-  uint64_t cN = pivot_word<kLA, kLX>(s, piv);
-  uint64_t mix = s.rmix;
-  uint32_t d = 0;
+  uint32_t piv = 0;
+  uint64_t cN = 0, mix = s.rmix;
+  int32_t d = -1;  // -1: the root itself is the node to decide
   while (true) {
-    if constexpr (kWL) {
-      if (wa.nodes - wa.last_poll >= pr.donate_check) {
-        wa.last_poll = wa.nodes;
-        heartbeat(pr, wa);
+    uint64_t Pn = cP, Xn = cX, En = cE, cmix = mix;
+    if (d >= 0) {
+      if constexpr (kWL) {
         clk.to(kBdQueue);
-        // only a task that has run for a while gives work away
-        wa.budget = __builtin_amdgcn_s_memrealtime() - wa.t_task >= pr.donate_age ? donation_budget(pr, wa) : 0;
+        poll_idle(pr, wa);
+        if (wa.budget > 0) {
+          if (donate_bits<kLA, kLX>(pr, s, (uint32_t)d, cP, cX, cE, piv, mix, wa)) wa.budget--;
+          else no_donation(pr, wa);
+        }
       }
-      if (wa.budget > 0) {
-        clk.to(kBdQueue);
-        if (donate_bits<kLA, kLX>(pr, s, d, cP, cX, cE, piv, mix, wa)) wa.budget--;
-        else wa.budget = 0;
+      clk.to(kBdSetOps);
+      const uint64_t B = cP & ~cN;
+      const uint64_t bm = ballot(B != 0);
+      if (bm == 0) {
+        if (d == 0) break;
+        clk.to(kBdBranch);
+        --d;
+        if ((uint32_t)d < s.lds_levels) frame_get<true>(s.fr_lds + (uint64_t)d * s.FS, W, WX, cP, cX, cE, piv, mix);
+        else frame_get<false>(s.fr_hbm + (uint64_t)(d - s.lds_levels) * s.FS, W, WX, cP, cX, cE, piv, mix);
+        cN = pivot_word<kLA, kLX>(s, piv);
+        continue;
       }
-    }
-    clk.to(kBdSetOps);
-    const uint64_t B = cP & ~cN;
-    const uint64_t bm = ballot(B != 0);
-    if (bm == 0) {
-      if (d == 0) break;
-      clk.to(kBdBranch);
-      --d;
-      if (d < s.lds_levels) frame_get<true>(s.fr_lds + (uint64_t)d * s.FS, W, WX, cP, cX, cE, piv, mix);
-      else frame_get<false>(s.fr_hbm + (uint64_t)(d - s.lds_levels) * s.FS, W, WX, cP, cX, cE, piv, mix);
-      cN = pivot_word<kLA, kLX>(s, piv);
-      continue;
-    }
-    const uint32_t k0 = ctz64(bm);
-    const uint32_t bit = ctz64(rdlane64(B, k0));
-    const uint32_t c = k0 * 64 + bit;
-    {
-      // c leaves P for X: one lane-select of the bit, then XOR (the bit is
-      // set in P) and OR
-      const uint64_t m = L == k0 ? (1ull << bit) : 0ull;
-      cP ^= m;
-      cX |= m;
-    }
-    const uint64_t Ac = act ? ld64<kLA>(s.A, (uint64_t)c * W + L) : 0;
-    const uint64_t Pn = cP & Ac, Xn = cX & Ac;
-    wa.nodes++;
-    const uint64_t cmix = mix + uniform64(ld64<kLA>(s.H, c));
-    const uint64_t pnz = ballot(Pn != 0);
-    if (pnz == 0) {
-      clk.to(kBdMaximal);
-      if (ballot(Xn != 0) == 0 && !rows_any<kLX>(s, cE, c)) report(pr, hist_lds, wa, s.rsize + d + 1, cmix);
-      continue;
-    }
-    const uint64_t En = filter_rows<kLX>(s, cE, c);
-    const uint64_t pnz2 = pnz & (pnz - 1);
-    if ((pnz2 & (pnz2 - 1)) == 0) {
-      // |P| <= 2 decided without the pivot scan, node for node as the scan
-      // would go (a pivot from X covering P leaves no child; ties go to the
-      // lowest index, inside X before outside rows)
-      const uint32_t k1 = ctz64(pnz);
-      const uint64_t w1 = rdlane64(Pn, k1);
-      const uint64_t w2 = pnz2 ? rdlane64(Pn, ctz64(pnz2)) : 0ull;
-      const uint32_t np = popc64(w1) + popc64(w2);
-      if (np == 1) {
-        // P = {a}: either an X vertex or outside row adjacent to a is the
-        // pivot and covers P, or a is the one child and a maximal clique
+      const uint32_t k0 = ctz64(bm);
+      const uint32_t bit = ctz64(rdlane64(B, k0));
+      const uint32_t c = k0 * 64 + bit;
+      {
+        // c leaves P for X: one lane-select of the bit, then XOR (the bit is
+        // set in P) and OR
+        const uint64_t m = L == k0 ? (1ull << bit) : 0ull;
+        cP ^= m;
+        cX |= m;
+      }
+      const uint64_t Ac = act ? ld64<kLA>(s.A, (uint64_t)c * W + L) : 0;
+      Pn = cP & Ac;
+      Xn = cX & Ac;
+      wa.nodes++;
+      cmix = mix + uniform64(ld64<kLA>(s.H, c));
+      const uint64_t pnz = ballot(Pn != 0);
+      if (pnz == 0) {
         clk.to(kBdMaximal);
-        const uint32_t na = k1 * 64 + ctz64(w1);
-        const uint64_t Aa = act ? ld64<kLA>(s.A, (uint64_t)na * W + L) : 0;
-        if (ballot((Xn & Aa) != 0) == 0 && !rows_any<kLX>(s, En, na)) {
+        if (ballot(Xn != 0) == 0 && !rows_any<kLX>(s, cE, c)) report(pr, hist_lds, wa, s.rsize + d + 1, cmix);
+        continue;
+      }
+      En = filter_rows<kLX>(s, cE, c);
+      const uint64_t pnz2 = pnz & (pnz - 1);
+      if ((pnz2 & (pnz2 - 1)) == 0) {
+        // |P| <= 2 decided without the pivot scan, node for node as the scan
+        // would go (a pivot from X covering P leaves no child; ties go to the
+        // lowest index, inside X before outside rows)
+        const uint32_t k1 = ctz64(pnz);
+        const uint64_t w1 = rdlane64(Pn, k1);
+        const uint64_t w2 = pnz2 ? rdlane64(Pn, ctz64(pnz2)) : 0ull;
+        const uint32_t np = popc64(w1) + popc64(w2);
+        if (np == 1) {
+          // P = {a}: either an X vertex or outside row adjacent to a is the
+          // pivot and covers P, or a is the one child and a maximal clique
+          clk.to(kBdMaximal);
+          const uint32_t na = k1 * 64 + ctz64(w1);
+          const uint64_t Aa = act ? ld64<kLA>(s.A, (uint64_t)na * W + L) : 0;
+          if (ballot((Xn & Aa) != 0) == 0 && !rows_any<kLX>(s, En, na)) {
+            wa.nodes++;
+            report(pr, hist_lds, wa, s.rsize + d + 2, cmix + uniform64(ld64<kLA>(s.H, na)));
+          }
+          continue;
+        }
+        if (np == 2) {
+          clk.to(kBdMaximal);
+          const uint32_t na = k1 * 64 + ctz64(w1);
+          const uint32_t nb = w2 ? (uint32_t)ctz64(pnz2) * 64 + ctz64(w2) : k1 * 64 + ctz64(w1 & (w1 - 1));
+          const uint64_t Aa = act ? ld64<kLA>(s.A, (uint64_t)na * W + L) : 0;
+          const uint64_t Ab = act ? ld64<kLA>(s.A, (uint64_t)nb * W + L) : 0;
+          const uint64_t Ea = filter_rows<kLX>(s, En, na), Eb = filter_rows<kLX>(s, En, nb);
+          const uint64_t Xa = Xn & Aa, Xb = Xn & Ab;
+          if (ballot(((Xa & Xb) | (Ea & Eb)) != 0)) continue;  // a pivot covers P
+          const uint64_t ha = uniform64(ld64<kLA>(s.H, na)), hb = uniform64(ld64<kLA>(s.H, nb));
+          if ((rdlane64(Aa, nb >> 6) >> (nb & 63)) & 1ull) {
+            // a ~ b: whichever pivot, the path is a then b (or b then a)
+            wa.nodes += 2;
+            report(pr, hist_lds, wa, s.rsize + d + 3, cmix + ha + hb);
+            continue;
+          }
+          const uint64_t xs = Xa | Xb, es = Ea | Eb;
+          const uint64_t xm = ballot(xs != 0), em = ballot(es != 0);
+          if (xm == 0 && em == 0) {
+            // all scores 0: children a and b, each a maximal clique
+            wa.nodes += 2;
+            report(pr, hist_lds, wa, s.rsize + d + 2, cmix + ha);
+            report(pr, hist_lds, wa, s.rsize + d + 2, cmix + hb);
+            continue;
+          }
+          // the pivot is the lowest X vertex (else outside row) adjacent to
+          // exactly one of a, b; the child is the other, maximal iff nothing
+          // in X or outside touches it
+          bool piv_a;
+          if (xm) {
+            const uint32_t k = ctz64(xm);
+            piv_a = (rdlane64(Xa, k) >> ctz64(rdlane64(xs, k))) & 1ull;
+          } else {
+            const uint32_t k = ctz64(em);
+            piv_a = (rdlane64(Ea, k) >> ctz64(rdlane64(es, k))) & 1ull;
+          }
           wa.nodes++;
-          report(pr, hist_lds, wa, s.rsize + d + 2, cmix + uniform64(ld64<kLA>(s.H, na)));
-        }
-        continue;
-      }
-      if (np == 2) {
-        clk.to(kBdMaximal);
-        const uint32_t na = k1 * 64 + ctz64(w1);
-        const uint32_t nb = w2 ? (uint32_t)ctz64(pnz2) * 64 + ctz64(w2) : k1 * 64 + ctz64(w1 & (w1 - 1));
-        const uint64_t Aa = act ? ld64<kLA>(s.A, (uint64_t)na * W + L) : 0;
-        const uint64_t Ab = act ? ld64<kLA>(s.A, (uint64_t)nb * W + L) : 0;
-        const uint64_t Ea = filter_rows<kLX>(s, En, na), Eb = filter_rows<kLX>(s, En, nb);
-        const uint64_t Xa = Xn & Aa, Xb = Xn & Ab;
-        if (ballot(((Xa & Xb) | (Ea & Eb)) != 0)) continue;  // a pivot covers P
-        const uint64_t ha = uniform64(ld64<kLA>(s.H, na)), hb = uniform64(ld64<kLA>(s.H, nb));
-        if ((rdlane64(Aa, nb >> 6) >> (nb & 63)) & 1ull) {
-          // a ~ b: whichever pivot, the path is a then b (or b then a)
-          wa.nodes += 2;
-          report(pr, hist_lds, wa, s.rsize + d + 3, cmix + ha + hb);
+          const uint64_t Xc = piv_a ? Xb : Xa, Ec = piv_a ? Eb : Ea;
+          if (ballot((Xc | Ec) != 0) == 0) report(pr, hist_lds, wa, s.rsize + d + 2, cmix + (piv_a ? hb : ha));
           continue;
         }
-        const uint64_t xs = Xa | Xb, es = Ea | Eb;
-        const uint64_t xm = ballot(xs != 0), em = ballot(es != 0);
-        if (xm == 0 && em == 0) {
-          // all scores 0: children a and b, each a maximal clique
-          wa.nodes += 2;
-          report(pr, hist_lds, wa, s.rsize + d + 2, cmix + ha);
-          report(pr, hist_lds, wa, s.rsize + d + 2, cmix + hb);
-          continue;
-        }
-        // the pivot is the lowest X vertex (else outside row) adjacent to
-        // exactly one of a, b; the child is the other, maximal iff nothing
-        // in X or outside touches it
-        bool piv_a;
-        if (xm) {
-          const uint32_t k = ctz64(xm);
-          piv_a = (rdlane64(Xa, k) >> ctz64(rdlane64(xs, k))) & 1ull;
-        } else {
-          const uint32_t k = ctz64(em);
-          piv_a = (rdlane64(Ea, k) >> ctz64(rdlane64(es, k))) & 1ull;
-        }
-        wa.nodes++;
-        const uint64_t Xc = piv_a ? Xb : Xa, Ec = piv_a ? Eb : Ea;
-        if (ballot((Xc | Ec) != 0) == 0) report(pr, hist_lds, wa, s.rsize + d + 2, cmix + (piv_a ? hb : ha));
-        continue;
       }
     }
-    if (small_ok<kWL>(pr, Pn, Xn, En)) {
-      solve_small<kWL, kStat, kLA, kLX>(pr, s, Pn, Xn, En, cmix, s.rsize + d + 1, hist_lds, wa, clk);
+    uint32_t np, nx;
+    if (small_ok<kWL>(pr, Pn, Xn, En, np, nx)) {
+      solve_small<kWL, kStat, kLA, kLX>(pr, s, Pn, Xn, En, np, nx, cmix, s.rsize + d + 1, hist_lds, wa, clk);
+      if (d < 0) break;
       continue;
     }
     uint32_t npiv, nbest;
     clk.to(kBdPivot);
     pick_pivot_bits<kLA, kLX>(s, Pn, Xn, En, npiv, nbest);
-    // (a pivot from X covering P needs no test here: the child level finds
-    // P & ~N(pivot) empty at once and backtracks, counting no node)
-    if (npiv == kNone) continue;
+    if (npiv == kNone || nbest == np) {  // nothing left, or a pivot that covers P
+      if (d < 0) break;
+      continue;
+    }
     clk.to(kBdBranch);
-    if (d < s.lds_levels) frame_put<true>(s.fr_lds + (uint64_t)d * s.FS, W, WX, cP, cX, cE, piv, mix);
-    else frame_put<false>(s.fr_hbm + (uint64_t)(d - s.lds_levels) * s.FS, W, WX, cP, cX, cE, piv, mix);
+    if (d >= 0) {
+      if ((uint32_t)d < s.lds_levels) frame_put<true>(s.fr_lds + (uint64_t)d * s.FS, W, WX, cP, cX, cE, piv, mix);
+      else frame_put<false>(s.fr_hbm + (uint64_t)(d - s.lds_levels) * s.FS, W, WX, cP, cX, cE, piv, mix);
+    }
     ++d;
     cP = Pn;
     cX = Xn;
@@ -2124,22 +2507,58 @@ __device__ __forceinline__ void solve_bits_t(const BkParams &pr, Sub &s, uint64_
   }
 }
 
+// A subproblem's own labels: tree nodes and cliques from here to end_task.
+__device__ __forceinline__ uint64_t begin_task(const Sub &s, WaveAcc &wa) {
+  wa.sub_cliques = 0;
+  wa.t_task = s.t0;
+  return wa.nodes;
+}
+__device__ __forceinline__ void end_task(const BkParams &pr, const Sub &s, const WaveAcc &wa, uint64_t nodes0) {
+  if (lane_id() == 0) {
+    if (pr.sub_nodes) atomicAdd(&pr.sub_nodes[s.root], (unsigned long long)(wa.nodes - nodes0));
+    if (pr.sub_cliques && wa.sub_cliques) atomicAdd(&pr.sub_cliques[s.root], (unsigned long long)wa.sub_cliques);
+  }
+}
+
+// solve_bits_t as a function of its own, one per placement.
+template <bool kWL, int kStat, bool kLA, bool kLX>
+__device__ __noinline__ __attribute__((not_tail_called)) void solve_bits_fn(ConstParams *kargs, uint32_t io, uint64_t cP, uint64_t cX,
+                                           uint64_t cE, uint32_t hist_lds_addr) {
+  const BkParams &pr = *(const BkParams *)(ConstParams *)uniform64((uint64_t)kargs);
+  LdsHandover *ho = handover(uniform(io));
+  const Sub s = lds_get(&ho->s);
+  WaveAcc wa = lds_get(&ho->w);
+  Clock<kStat> clk;
+  const uint64_t nodes0 = begin_task(s, wa);
+  solve_bits_t<kWL, kStat, kLA, kLX>(pr, s, cP, cX, cE,
+                                     (lds_ull *)(uintptr_t)uniform(hist_lds_addr), wa, clk);
+  end_task(pr, s, wa, nodes0);
+  lds_put(&ho->w, wa);
+}
+
+// (s is in the hand-over block already where the kernel uses functions)
 template <bool kWL, int kStat>
 __device__ __forceinline__ void solve_bits(const BkParams &pr, Sub &s, uint64_t cP, uint64_t cX, uint64_t cE,
-                                           unsigned long long *hist_lds, WaveAcc &wa, Clock<kStat> &clk) {
+                                           lds_ull *hist_lds, WaveAcc &wa, Clock<kStat> &clk) {
+  if constexpr (fn_of(true, kStat)) {
+    ConstParams *ka = (ConstParams *)__builtin_amdgcn_kernarg_segment_ptr();
+    const uint32_t ha = (uint32_t)(uintptr_t)hist_lds;
+    if (s.where == 3) solve_bits_fn<kWL, kStat, true, true>(ka, wa.io, cP, cX, cE, ha);
+    else if (s.where == 1) solve_bits_fn<kWL, kStat, true, false>(ka, wa.io, cP, cX, cE, ha);
+    else solve_bits_fn<kWL, kStat, false, false>(ka, wa.io, cP, cX, cE, ha);
+    return;
+  }
+  const uint64_t nodes0 = begin_task(s, wa);
   if (s.where == 3) solve_bits_t<kWL, kStat, true, true>(pr, s, cP, cX, cE, hist_lds, wa, clk);
   else if (s.where == 1) solve_bits_t<kWL, kStat, true, false>(pr, s, cP, cX, cE, hist_lds, wa, clk);
   else solve_bits_t<kWL, kStat, false, false>(pr, s, cP, cX, cE, hist_lds, wa, clk);
-  // the subproblem's counts are complete once its queued subtrees have run
-  if constexpr (lane_of(kStat)) {
-    clk.to(kBdSetOps);
-    ls_flush(pr, hist_lds, wa);
-  }
+  clk.to(kBdOther);
+  end_task(pr, s, wa, nodes0);
 }
 
 // Intersection of ascending a[0,na) and b[0,nb) written to out (ascending);
 // iterates the shorter list and binary-searches the longer.
-__device__ __forceinline__ uint32_t intersect_into(const uint32_t *a, uint32_t na, const uint32_t *b, uint32_t nb, uint32_t *out) {
+__device__ __forceinline__ uint32_t intersect_in(const uint32_t *a, uint32_t na, const uint32_t *b, uint32_t nb, uint32_t *out) {
   if (na > nb) {
     const uint32_t *t = a;
     a = b;
@@ -2164,6 +2583,17 @@ __device__ __forceinline__ uint32_t intersect_into(const uint32_t *a, uint32_t n
   }
   return w;
 }
+__device__ __noinline__ __attribute__((not_tail_called)) uint32_t intersect_fn(const uint32_t *a, uint32_t na,
+                                                                               const uint32_t *b, uint32_t nb,
+                                                                               uint32_t *out) {
+  return intersect_in((const uint32_t *)uniform64((uint64_t)a), uniform(na), (const uint32_t *)uniform64((uint64_t)b),
+                      uniform(nb), out);
+}
+template <bool kFn>
+__device__ __forceinline__ uint32_t intersect_into(const uint32_t *a, uint32_t na, const uint32_t *b, uint32_t nb, uint32_t *out) {
+  if constexpr (!kFn) return intersect_in(a, na, b, nb, out);
+  return uniform(intersect_fn(a, na, b, nb, out));
+}
 
 
 __device__ __forceinline__ uint32_t hw_cu_id() {
@@ -2184,41 +2614,93 @@ __device__ __forceinline__ void defer(const BkParams &pr, uint64_t it) {
 }
 
 
-template <bool kIPX, bool kWL, int kStat>
-__device__ __forceinline__ void finish_sub(const BkParams &pr, Sub &s, uint64_t P0, uint64_t X0, unsigned long long *hist_lds,
-                           WaveAcc &wa, Clock<kStat> &clk) {
-  const uint64_t nodes0 = wa.nodes;
-  clk.to(kBdInduced);
-  build<kIPX>(pr, s);
-  bk_solve<kIPX, kWL, kStat>(pr, s, P0, X0, hist_lds, wa, clk);
-  clk.to(kBdOther);
-  if (lane_id() == 0) {
-    if (pr.sub_nodes) atomicAdd(&pr.sub_nodes[s.root], (unsigned long long)(wa.nodes - nodes0));
-    if (pr.sub_cliques && wa.sub_cliques) atomicAdd(&pr.sub_cliques[s.root], (unsigned long long)wa.sub_cliques);
+// The list path: builds the rows (a received task has them) and solves.
+template <bool kIPX, bool kWL, int kStat, bool kBuild>
+__device__ __noinline__ __attribute__((not_tail_called)) void solve_list_fn(ConstParams *kargs, uint32_t io, uint64_t cP, uint64_t cX,
+                                           uint32_t hist_lds_addr) {
+  const BkParams &pr = *(const BkParams *)(ConstParams *)uniform64((uint64_t)kargs);
+  LdsHandover *ho = handover(uniform(io));
+  Sub s = lds_get(&ho->s);
+  WaveAcc wa = lds_get(&ho->w);
+  Clock<kStat> clk;
+  const uint64_t nodes0 = begin_task(s, wa);
+  if constexpr (kBuild) build<kIPX>(pr, s);
+  bk_solve<kIPX, kWL, kStat>(pr, s, cP, cX, (lds_ull *)(uintptr_t)uniform(hist_lds_addr), wa, clk);
+  end_task(pr, s, wa, nodes0);
+  lds_put(&ho->w, wa);
+}
+template <bool kIPX, bool kWL, int kStat, bool kBuild>
+__device__ __forceinline__ void solve_list(const BkParams &pr, Sub &s, uint64_t cP, uint64_t cX,
+                                           lds_ull *hist_lds, WaveAcc &wa, Clock<kStat> &clk) {
+  if constexpr (fn_of(kIPX, kStat)) {
+    lds_put(&handover(wa.io)->s, s);
+    solve_list_fn<kIPX, kWL, kStat, kBuild>((ConstParams *)__builtin_amdgcn_kernarg_segment_ptr(), wa.io, cP, cX,
+                                            (uint32_t)(uintptr_t)hist_lds);
+    return;
   }
+  const uint64_t nodes0 = begin_task(s, wa);
+  clk.to(kBdInduced);
+  if constexpr (kBuild) build<kIPX>(pr, s);
+  bk_solve<kIPX, kWL, kStat>(pr, s, cP, cX, hist_lds, wa, clk);
+  clk.to(kBdOther);
+  end_task(pr, s, wa, nodes0);
 }
 
 template <bool kWL, int kStat>
 __device__ __forceinline__ void finish_bits(const BkParams &pr, Sub &s, const uint32_t *ids, uint32_t q0, bool filter,
-                                            uint64_t keep, unsigned long long *hist_lds, WaveAcc &wa,
+                                            uint64_t keep, lds_ull *hist_lds, WaveAcc &wa,
                                             Clock<kStat> &clk) {
-  const uint64_t nodes0 = wa.nodes;
   clk.to(kBdInduced);
-  const uint64_t E0 = build_bits(pr, s, ids, q0, keep, filter);
+  lds_put(&handover(wa.io)->s, s);
+  const uint64_t E0 =
+      build_bits_fn((ConstParams *)__builtin_amdgcn_kernarg_segment_ptr(), wa.io, ids, q0, keep, filter);
   solve_bits<kWL, kStat>(pr, s, full_word(s.p), 0, E0, hist_lds, wa, clk);
-  clk.to(kBdOther);
-  if (lane_id() == 0) {
-    if (pr.sub_nodes) atomicAdd(&pr.sub_nodes[s.root], (unsigned long long)(wa.nodes - nodes0));
-    if (pr.sub_cliques && wa.sub_cliques) atomicAdd(&pr.sub_cliques[s.root], (unsigned long long)wa.sub_cliques);
-  }
+}
+
+// The kernel's arguments, read again: values read before are not carried over
+// the calls in between (which use all registers, so that they were stored to
+// scratch memory and read back, 100 registers a subproblem).
+template <bool kFn>
+__device__ __forceinline__ const BkParams &fresh_params(const BkParams &args) {
+  if constexpr (!kFn) return args;
+  ConstParams *k = (ConstParams *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(k));
+  return *(const BkParams *)k;
+}
+// A subproblem of wave gw with nothing but the graph set.
+__device__ __forceinline__ Sub fresh_sub(const BkParams &pr, uint32_t gw) {
+  Sub s{};
+  s.oc = pr.oc;
+  s.rp = pr.rp;
+  s.split = pr.split;
+  s.cover = pr.cover + (uint64_t)gw * kWave;
+  return s;
+}
+
+// Runs what is left in the wave's lane queue.
+template <int kStat>
+__device__ __noinline__ __attribute__((not_tail_called)) void ls_flush_fn(ConstParams *kargs, uint32_t io,
+                                                                          uint32_t hist_lds_addr) {
+  const BkParams &pr = *(const BkParams *)(ConstParams *)uniform64((uint64_t)kargs);
+  LdsHandover *ho = handover(uniform(io));
+  WaveAcc wa = lds_get(&ho->w);
+  ls_flush<kStat>(pr, (lds_ull *)(uintptr_t)uniform(hist_lds_addr), wa);
+  lds_put(&ho->w, wa);
+}
+template <int kStat>
+__device__ __forceinline__ void finish_lanes(lds_ull *hist_lds, const WaveAcc &wa) {
+  if constexpr (lane_of(kStat))
+    ls_flush_fn<kStat>((ConstParams *)__builtin_amdgcn_kernarg_segment_ptr(), wa.io, (uint32_t)(uintptr_t)hist_lds);
 }
 
 template <bool kIPX, bool kWL, int kStat>
 // At least four waves per SIMD (<= 128 VGPRs): occupancy hides the LDS and
 // memory latency of the set operations better than registers would.
-__global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) void bk_kernel(BkParams pr) {
+__global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) void bk_kernel(BkParams args) {
+  constexpr bool kFn = fn_of(kIPX, kStat);
+  const BkParams &pr = args;
   extern __shared__ __align__(16) uint8_t smem[];
-  unsigned long long *hist_lds = (unsigned long long *)smem;
+  lds_ull *hist_lds = (lds_ull *)smem;
   const uint32_t wig = threadIdx.x / kWave, L = lane_id();
   const uint32_t hb = (uint32_t)align8(8ull * pr.hist_lds);
   Pool pl;
@@ -2237,21 +2719,18 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
   const uint32_t gw = blockIdx.x * pr.wpg + wig;
   uint8_t *hbm = pr.hbm + (uint64_t)gw * pr.hbm_bytes;
   WaveAcc wa;
+  wa.io = (uint32_t)(uintptr_t)(smem + pr.io_off + wig * kHandoverBytes);
   if (lane_of(kStat)) {
-    wa.ls_lds = (uint32_t)(uintptr_t)(smem + pr.ls_off + wig * kLsBytes);
-    wa.ls_h = pr.ls_h + (uint64_t)gw * (kLsGlobalBytes / 8);
+    wa.ls = pr.ls + (uint64_t)gw * kLsBytes;
+    wa.ls_lds = (uint32_t)(uintptr_t)(smem + pr.ls_off + wig * kLsLds);
   }
   wa.xq = (hw_cu_id() >> 8) % kQueues;
   wa.peek = wa.xq;
   Clock<kStat> clk;
   clk.start();
-  Sub s;
-  s.oc = pr.oc;
-  s.rp = pr.rp;
-  s.split = pr.split;
-  s.cover = pr.cover + (uint64_t)gw * kWave;
-  const uint32_t *items1 = (const uint32_t *)pr.items;
-  const uint2 *items2 = (const uint2 *)pr.items;
+  // the totals live in the hand-over block while functions solve; of `wa`,
+  // only io and xq are then used between here and the end
+  if constexpr (kFn) lds_put(&handover(wa.io)->w, wa);
   // phase 1: first-level subproblems by ticket. A wave's first ticket is its
   // position in the grid (neighbouring tickets, the heaviest, on different
   // workgroups, so that they do not share a CU's LDS pool), the next ones
@@ -2260,6 +2739,7 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
   const uint32_t nwaves = gridDim.x * pr.wpg;
   uint32_t tickets = 0;
   while (true) {
+    const BkParams &pr = fresh_params<kFn>(args);
     clk.to(kBdQueue);
     uint32_t t = wig * gridDim.x + blockIdx.x;
     if (tickets) {
@@ -2279,12 +2759,16 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
       hi = lo + pr.chunk;
     }
     if (lo >= pr.n_items) break;
-    hi = min(hi, pr.n_items);
+    lo = uniform64(lo);
+    hi = uniform64(min(hi, pr.n_items));
     ++tickets;
     clk.to(kBdInduced);
     for (uint64_t it = lo; it < hi; ++it) {
-      wa.sub_cliques = 0;
-      wa.t_task = __builtin_amdgcn_s_memrealtime();
+      const BkParams &pr = fresh_params<kFn>(args);
+      const uint32_t *items1 = (const uint32_t *)pr.items;
+      const uint2 *items2 = (const uint2 *)pr.items;
+      Sub s = fresh_sub(pr, gw);
+      s.t0 = __builtin_amdgcn_s_memrealtime();
       // level 1: vertex items; level 2: arc items; level 3: arc items where
       // (v, kNone) stands for the whole vertex subproblem of v
       bool vertex_item = pr.level == 1;
@@ -2315,21 +2799,21 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
         uint32_t qb = q;
         bool filter = false;
         if (kIPX && !bits) {
-          qb = live_count(pr, pr.oc + s0, p, pr.oc + b0, q, s.cover);
+          qb = live_count(pr.oc + s0, p, pr.oc + b0, q, s.cover);
           bits = filter = qb <= kMaxXRows;
           if (!bits) qb = q;
         }
         const uint64_t keep = !bits || filter ? 0ull
-                              : q > 2 * p     ? live_rows(pr, pr.oc + s0, p, pr.oc + b0, q, qb)
+                              : q > 2 * p     ? live_rows(pr.oc + s0, p, pr.oc + b0, q, qb)
                                               : all_rows(q);
-        const Region rg = bits ? pool_take_wait(pl, bits_want(p, qb, W, lv), bits_want_inner(p, qb, W, lv),
+        const Region rg = bits ? pool_take_wait<kFn>(pl, bits_want(p, qb, W, lv), bits_want_inner(p, qb, W, lv),
                                                 bits_fs(W, (qb + 63) / 64) * min(p, lv),
                                                 bits_want_inner(p, qb, W, lv))
-                               : pool_take_wait(pl, list_want(p, q, W, kIPX, lv), 0, (16 * W + 16) * min(p, lv),
+                               : pool_take_wait<kFn>(pl, list_want(p, q, W, kIPX, lv), 0, (16 * W + 16) * min(p, lv),
                                                 list_want(p, q, W, kIPX, lv));
         if (!(bits ? place_bits(s, p, qb, W, rg.ptr, rg.bytes, hbm, pr.hbm_bytes, pr.stack_lds)
                    : place(s, p, q, W, kIPX, rg.ptr, rg.bytes, hbm, pr.hbm_bytes, pr.stack_lds))) {
-          pool_put(pl, rg);
+          pool_put<kFn>(pl, rg);
           defer(pr, it);
           continue;
         }
@@ -2344,9 +2828,9 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
           finish_bits<kWL, kStat>(pr, s, pr.oc + b0, q, filter, keep, hist_lds, wa, clk);
         } else {
           for (uint32_t i = L; i < q; i += kWave) s.XL[i] = pr.oc[b0 + i];
-          finish_sub<kIPX, kWL, kStat>(pr, s, full_word(p), 0, hist_lds, wa, clk);
+          solve_list<kIPX, kWL, kStat, true>(pr, s, full_word(p), 0, hist_lds, wa, clk);
         }
-        pool_put(pl, rg);
+        pool_put<kFn>(pl, rg);
       } else {
         const uint32_t u = ia.x, w = ia.y;
         const uint64_t su = pr.split[u], eu = pr.rp[u + 1], bu = pr.rp[u];
@@ -2354,30 +2838,39 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
         const uint32_t pb = (uint32_t)min(eu - su, ew - sw), qb = (uint32_t)min(eu - bu, sw - bw);
         Sub t = s;
         const uint32_t Wb = (pb + 63) / 64;
-        const Region rg = pool_take_wait(pl, list_want(pb, qb, Wb, kIPX, lv), 0, (16 * Wb + 16) * min(pb, lv),
+        const Region rg = pool_take_wait<kFn>(pl, list_want(pb, qb, Wb, kIPX, lv), 0, (16 * Wb + 16) * min(pb, lv),
                                          list_want(pb, qb, Wb, kIPX, lv));
         if (!place(t, pb, qb, Wb, kIPX, rg.ptr, rg.bytes, hbm, pr.hbm_bytes, pr.stack_lds)) {
-          pool_put(pl, rg);
+          pool_put<kFn>(pl, rg);
           defer(pr, it);
           continue;
         }
-        const uint32_t p = intersect_into(pr.oc + su, (uint32_t)(eu - su), pr.oc + sw, (uint32_t)(ew - sw), t.S);
-        const uint32_t q = intersect_into(pr.ci + bu, (uint32_t)(eu - bu), pr.oc + bw, (uint32_t)(sw - bw), t.XL);
+        const uint32_t p = intersect_into<kFn>(pr.oc + su, (uint32_t)(eu - su), pr.oc + sw, (uint32_t)(ew - sw), t.S);
+        const uint32_t q = intersect_into<kFn>(pr.ci + bu, (uint32_t)(eu - bu), pr.oc + bw, (uint32_t)(sw - bw), t.XL);
         const uint64_t rmix = splitmix64(u) + splitmix64(w);
         if (p == 0) {
-          if (q == 0) report(pr, hist_lds, wa, 2, rmix);
-          if (pr.sub_cliques && L == 0 && wa.sub_cliques) atomicAdd(&pr.sub_cliques[u], wa.sub_cliques);
-          pool_put(pl, rg);
+          if (q == 0) {
+            LdsHandover *ho = handover(wa.io);
+            if constexpr (kFn) {
+              WaveAcc w = lds_get(&ho->w);
+              report(pr, hist_lds, w, 2, rmix);
+              lds_put(&ho->w, w);
+            } else {
+              report(pr, hist_lds, wa, 2, rmix);
+            }
+            if (pr.sub_cliques && L == 0) atomicAdd(&pr.sub_cliques[u], 1ull);
+          }
+          pool_put<kFn>(pl, rg);
           continue;
         }
         // re-lay the arena for the actual sizes (and, bitmap path, the kept rows)
         const uint32_t W = (p + 63) / 64;
         const bool bits = kIPX && q <= kMaxXRows;
         uint32_t qk = q;
-        const uint64_t keep = !bits ? 0ull : q > 2 * p ? live_rows(pr, t.S, p, t.XL, q, qk) : all_rows(q);
+        const uint64_t keep = !bits ? 0ull : q > 2 * p ? live_rows(t.S, p, t.XL, q, qk) : all_rows(q);
         if (!(bits ? place_bits(s, p, qk, W, rg.ptr, rg.bytes, hbm, pr.hbm_bytes, pr.stack_lds)
                    : place(s, p, q, W, kIPX, rg.ptr, rg.bytes, hbm, pr.hbm_bytes, pr.stack_lds))) {
-          pool_put(pl, rg);
+          pool_put<kFn>(pl, rg);
           defer(pr, it);
           continue;
         }
@@ -2392,14 +2885,16 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
         s.root = u;
         s.rmix = rmix;
         if (bits) finish_bits<kWL, kStat>(pr, s, t.XL, q, false, keep, hist_lds, wa, clk);
-        else finish_sub<kIPX, kWL, kStat>(pr, s, full_word(p), 0, hist_lds, wa, clk);
-        pool_put(pl, rg);
+        else solve_list<kIPX, kWL, kStat, true>(pr, s, full_word(p), 0, hist_lds, wa, clk);
+        pool_put<kFn>(pl, rg);
       }
     }
   }
+  clk.to(kBdSetOps);
+  finish_lanes<kStat>(hist_lds, wa);
   // (the launch cannot end before this wave gets here: its tickets leave the
   // outstanding count together)
-  if (kWL && L == 0 && tickets) atomicSub(pr.ctl + kCtlOutstanding, (unsigned long long)tickets);
+  if (kWL && tickets) tasks_done(pr, tickets);
   // phase 2: donated subtrees until no work is outstanding. An idle wave puts
   // itself on the idle queue and waits on its own mailbox line; a donor takes
   // it off the queue and writes the task into its slot, so no line is polled
@@ -2417,9 +2912,15 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
       if (!registered) registered = register_idle(pr, gw, wa.xq);
       if (registered) {
         const unsigned long long got = uniform64(L == 0 ? ld_relaxed(&pr.mbox[(uint64_t)gw * kMboxStride]) : 0ull);
+        if (got == kMboxDone) break;
         if (got) {
+          const BkParams &pr = fresh_params<kFn>(args);
+          Sub s = fresh_sub(pr, gw);
           registered = false;
           backoff = 1;
+          // (empty again before this wave can be registered again; it stays
+          // empty until then, with this task outstanding)
+          if (L == 0) st_shared(&pr.mbox[(uint64_t)gw * kMboxStride], 0ull);
           drain();
           const uint64_t *h = (const uint64_t *)slot;
           const uint64_t h0 = uniform64(ld_shared(h)), h1 = uniform64(ld_shared(h + 1)), h2 = uniform64(ld_shared(h + 2)),
@@ -2429,7 +2930,7 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
           if (kIPX && kind == kTaskBits) {
             const bool shape = p <= pr.slot_pmax && W == (p + 63) / 64 && nx <= pr.slot_xcap && nx <= kMaxXRows;
             if (shape)
-              rsv = pool_take_wait(pl, bits_want(p, nx, W, lv), bits_want_inner(p, nx, W, lv),
+              rsv = pool_take_wait<kFn>(pl, bits_want(p, nx, W, lv), bits_want_inner(p, nx, W, lv),
                                    bits_fs(W, (nx + 63) / 64) * min(p, lv), bits_want_inner(p, nx, W, lv));
             const Region rg = rsv;
             const bool okb = shape && place_bits(s, p, nx, W, rg.ptr, rg.bytes, hbm, pr.hbm_bytes, pr.stack_lds);
@@ -2455,28 +2956,22 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
               s.rsize = rsize;
               s.root = root;
               s.rmix = rmix;
-              wa.sub_cliques = 0;
-              wa.t_task = __builtin_amdgcn_s_memrealtime();
-              const uint64_t nodes0 = wa.nodes;
+              s.t0 = __builtin_amdgcn_s_memrealtime();
+              if constexpr (kFn) lds_put(&handover(wa.io)->s, s);
               solve_bits<kWL, kStat>(pr, s, P0, X0, E0, hist_lds, wa, clk);
-              clk.to(kBdOther);
-              if (L == 0) {
-                if (pr.sub_nodes) atomicAdd(&pr.sub_nodes[root], (unsigned long long)(wa.nodes - nodes0));
-                if (pr.sub_cliques && wa.sub_cliques)
-                  atomicAdd(&pr.sub_cliques[root], (unsigned long long)wa.sub_cliques);
-              }
+              finish_lanes<kStat>(hist_lds, wa);  // before the task counts as done
             } else if (L == 0) {
               atomicOr(&pr.acc[kAccError], 2ull);
             }
-            if (L == 0) atomicSub(pr.ctl + kCtlOutstanding, 1ull);
-            pool_put(pl, rsv);
+            tasks_done(pr, 1);
+            pool_put<kFn>(pl, rsv);
             rsv = Region{pl.base, 0, 0, 0};
             t0 = __builtin_amdgcn_s_memrealtime();
             continue;
           }
           const bool shape = kind == kTaskList && p <= pr.slot_pmax && W == (p + 63) / 64 && nx <= pr.slot_xcap;
           if (shape)
-            rsv = pool_take_wait(pl, list_want(p, nx, W, kIPX, lv), 0, (16 * W + 16) * min(p, lv),
+            rsv = pool_take_wait<kFn>(pl, list_want(p, nx, W, kIPX, lv), 0, (16 * W + 16) * min(p, lv),
                                  list_want(p, nx, W, kIPX, lv));
           const Region rg = rsv;
           const bool ok = shape && place(s, p, nx, W, kIPX, rg.ptr, rg.bytes, hbm, pr.hbm_bytes, pr.stack_lds);
@@ -2507,20 +3002,13 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
             s.rsize = rsize;
             s.root = root;
             s.rmix = rmix;
-            wa.sub_cliques = 0;
-            wa.t_task = __builtin_amdgcn_s_memrealtime();
-            const uint64_t nodes0 = wa.nodes;
-            bk_solve<kIPX, kWL, kStat>(pr, s, P0, X0, hist_lds, wa, clk);
-            clk.to(kBdOther);
-            if (L == 0) {
-              if (pr.sub_nodes) atomicAdd(&pr.sub_nodes[root], (unsigned long long)(wa.nodes - nodes0));
-              if (pr.sub_cliques && wa.sub_cliques) atomicAdd(&pr.sub_cliques[root], (unsigned long long)wa.sub_cliques);
-            }
+            s.t0 = __builtin_amdgcn_s_memrealtime();
+            solve_list<kIPX, kWL, kStat, false>(pr, s, P0, X0, hist_lds, wa, clk);
           } else if (L == 0) {
             atomicOr(&pr.acc[kAccError], 2ull);  // donors only publish what fits
           }
-          if (L == 0) atomicSub(pr.ctl + kCtlOutstanding, 1ull);
-          pool_put(pl, rsv);
+          tasks_done(pr, 1);
+          pool_put<kFn>(pl, rsv);
           rsv = Region{pl.base, 0, 0, 0};
           t0 = __builtin_amdgcn_s_memrealtime();
           continue;
@@ -2546,9 +3034,10 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
       for (uint32_t z = 0; z < backoff; ++z) __builtin_amdgcn_s_sleep(32);
       backoff = min(backoff * 2, registered ? 16u : 64u);
     }
-    pool_put(pl, rsv);
+    pool_put<kFn>(pl, rsv);
   }
   clk.to(kBdOther);
+  if constexpr (kFn) wa = lds_get(&handover(wa.io)->w);
   if (L == 0) {
     if (pr.wave_val) {
       pr.wave_val[gw] = kStat == kStatDonor ? wa.donations : wa.nodes;
@@ -2559,6 +3048,8 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
         for (int i = 0; i < 7; ++i) pr.wave_bd[(uint64_t)gw * 7 + i] = clk.acc[i];
     }
   }
+  wa.count += wa.ls_count;
+  wa.nodes += wa.ls_nodes;
   // totals: summed over the workgroup in the pool's mask words (the pool is
   // done), one update each and workgroup (five by every wave, on one line,
   // were 0.2 ms of every launch)
@@ -2579,7 +3070,7 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
   if (threadIdx.x < 4 && tot[threadIdx.x]) atomicAdd(&pr.acc[threadIdx.x], tot[threadIdx.x]);
   if (threadIdx.x == 4 && tot[4] > ld_relaxed(&pr.acc[kAccMaxSize])) atomicMax(&pr.acc[kAccMaxSize], tot[4]);
   for (uint32_t i = threadIdx.x; i < pr.hist_lds; i += blockDim.x)
-    if (hist_lds[i]) atomicAdd(&pr.hist[min(i, pr.hist_len - 1)], hist_lds[i]);
+    if (const unsigned long long h = hist_lds[i]) atomicAdd(&pr.hist[min(i, pr.hist_len - 1)], h);
 }
 
 __global__ void reset_kernel(unsigned long long *acc, uint32_t n, uint32_t *ticket) {
@@ -2783,7 +3274,7 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
   int cus = 0;
   MCE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   // the lane solver runs in its own kernel instance (IPX, no statistics)
-  const uint32_t ls_max = stat_of(cfg.task) == kStatNone && cfg.ipx ? std::min<uint32_t>(cfg.lane_max, kLsMax) : 0;
+  const uint32_t ls_max = stat_of(cfg.task) == kStatNone && cfg.ipx ? std::min<uint32_t>(cfg.lane_max, kLsP + kLsX) : 0;
   const int stat = ls_max ? kStatLane : stat_of(cfg.task);
   const uint32_t hist_lds = std::min<uint32_t>(hist_len, 128);
   const size_t hist_bytes = (8ull * hist_lds + 7) & ~7ull;
@@ -2799,19 +3290,20 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
     BkParams probe{};
     int rc0 = dispatch(cfg.ipx, cfg.wl, stat, true, &nb_regs, probe, 0, 4, hist_bytes + kPoolHeader + 4096, s);
     if (rc0) return rc0;
-    const uint32_t waves_cu = 4 * (uint32_t)std::max(nb_regs, 1);
+    // (never more than the four waves per SIMD that buffers and pools are
+    // sized for, also where an instance needs fewer registers)
+    const uint32_t waves_cu = 4 * std::min((uint32_t)std::max(nb_regs, 1), waves_per_simd_of(cfg.wl));
     groups_cu = std::max<uint32_t>(groups_cu, (waves_cu + max_wpg - 1) / max_wpg);
     wpg = std::max<uint32_t>(1, waves_cu / groups_cu);
   }
   wpg = std::max<uint32_t>(1, std::min<uint32_t>(wpg, max_wpg));
-  // the lane solver's regions (one per wave) follow the pool, 64-byte aligned
-  const size_t ls_total = ls_max ? (size_t)kLsBytes * wpg + 64 : 0;
+  // the waves' hand-over blocks and the lane solver's LDS parts follow the pool
+  const size_t ls_total = (kHandoverBytes + (ls_max ? (size_t)kLsLds : 0)) * wpg;
   const size_t fixed = hist_bytes + kPoolHeader + ls_total, share = lds_cu / groups_cu;
   size_t pool = cfg.lds_bytes ? (size_t)cfg.lds_bytes * wpg : share > fixed + kGranule ? share - fixed : kGranule;
   pool = std::min<size_t>(pool, lds_cu - fixed);
   pool = std::min<size_t>(pool, (size_t)kPoolWords * 64 * kGranule) / kGranule * kGranule;
-  const size_t ls_off = ls_max ? (hist_bytes + kPoolHeader + pool + 63) & ~(size_t)63 : 0;
-  const size_t lds = ls_max ? ls_off + (size_t)kLsBytes * wpg : hist_bytes + kPoolHeader + pool;
+  const size_t lds = fixed + pool;
   if (lds > lds_cu) return set_error(MCE_EINVAL, "LDS per workgroup %zu exceeds 160 KiB", lds);
 
   // every device buffer of this call: carved from the caller's scratch
@@ -2918,8 +3410,8 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
   unsigned long long *wave_val = nullptr, *wave_bd = nullptr;
   uint32_t *wave_cu = nullptr;
   if (arena && (rc = dmalloc((void **)&hbm, arena * waves, kWsArena))) return rc;
-  uint64_t *ls_h = nullptr;
-  if (ls_max && (rc = dmalloc((void **)&ls_h, (uint64_t)kLsGlobalBytes * waves, kWsLane))) return rc;
+  uint8_t *ls = nullptr;
+  if (ls_max && (rc = dmalloc((void **)&ls, (uint64_t)kLsBytes * waves, kWsLane))) return rc;
   if (cover && waves > max_waves) return set_error(MCE_EINTERNAL, "%u waves exceed the hub filter's %u", waves, max_waves);
   if (hneed[1] && (rc = dmalloc((void **)&overflow, sizeof(uint64_t) * hneed[1], kWsOverflow))) return rc;
   if (wave_stats) {
@@ -2944,8 +3436,9 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
   pr.small_max = std::min<uint32_t>(cfg.small_max, kSmallMax);
   pr.small_pmax = kSmallMaxPWl;
   pr.ls_max = ls_max;
-  pr.ls_off = (uint32_t)ls_off;
-  pr.ls_h = ls_h;
+  pr.io_off = (uint32_t)(hist_bytes + kPoolHeader + pool);
+  pr.ls_off = pr.io_off + kHandoverBytes * wpg;
+  pr.ls = ls;
   pr.cover = cover;
   pr.watchdog_ticks = cfg.watchdog_us ? (uint64_t)cfg.watchdog_us * 100 : kWatchdogTicks;
   pr.hbm = hbm;
@@ -2979,6 +3472,8 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
     pr.donate_min_p = std::max<uint32_t>(cfg.donate_min_p, 1);
     pr.donate_check = std::max<uint32_t>(cfg.donate_check_nodes, 1);
     pr.donate_age = (uint64_t)cfg.donate_age_us * 100;
+    // looks at the idle queues at least 20 us apart, or the age if less
+    pr.poll_ticks = cfg.donate_auto ? 2000 : std::min<uint64_t>(2000, pr.donate_age);
     if ((rc = dmalloc((void **)&pr.ctl, sizeof(unsigned long long) * kCtlWords, kWsCtl))) return rc;
     if ((rc = dmalloc((void **)&pr.seq, sizeof(unsigned long long) * kQueues * pr.ring_cap, kWsSeq))) return rc;
     if ((rc = dmalloc((void **)&pr.ring, pr.slot_bytes * pr.ring_cap, kWsRing))) return rc;

@@ -56,7 +56,7 @@ enum WsSlot : int {
   kWsRing,
   kWsIdle,
   kWsMbox,
-  kWsLane,      // lane solver: hash terms, headers and frames of every wave
+  kWsLane,      // lane solver: slots, hash terms and frames of every wave
   kWsCover,     // hub row filter: 64 words per wave
   kWsSlots
 };
@@ -100,6 +100,10 @@ struct Scratch {
 int schedule_by_key(const DevGraph &g, const uint32_t *key, uint32_t key_max, uint32_t *order,
                     uint32_t *len_out, hipStream_t s, Scratch *sc = nullptr);
 
+// Largest lane-solver subtree when the caller leaves it to the engine: every
+// one that its registers hold (15 members of P, 48 of X).
+constexpr uint32_t kLaneAuto = 63;
+
 struct BkLaunch {
   int level = 1;       // 1 = vertex subproblems, 2 = arc subproblems, 3 = both (mixed list)
   bool ipx = true;
@@ -113,8 +117,9 @@ struct BkLaunch {
   uint32_t donate_min_p = 10;
   uint32_t donate_check_nodes = 64;
   uint32_t donate_age_us = 1000;
+  bool donate_auto = false;  // the caller left the donation thresholds, and with them the rhythm, to the engine
   uint32_t small_max = 64;  // P + X + outside rows at which a node goes to the small-universe solver (0 = never)
-  uint32_t lane_max = 16;   // P + X at which the small-universe solver queues a subtree for the lane solver (0 = never)
+  uint32_t lane_max = kLaneAuto;  // P + X at which the small-universe solver queues a subtree for the lane solver (0 = never)
   uint32_t watchdog_us = 0;  // worker list: idle time without global progress before giving up (0 = 120 s)
   uint32_t progress_s = 0;   // > 0: print the launch's own progress counters to stderr this often
   bool capture = false;  // run the enumeration launch as a captured hipGraph
