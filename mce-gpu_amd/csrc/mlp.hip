@@ -119,16 +119,29 @@ __global__ __launch_bounds__(256) void features_kernel(uint32_t n, const uint64_
 struct TrainArgs {
   const float *x;       // rows x 16
   const float *y;       // rows
-  const uint32_t *idx;  // rows of this step
+  const uint32_t *idx;  // rows of this step (null: all, in order)
   uint32_t nrows;
   float inv_batch;      // 1 / rows of the step
   const float *params;  // kP
   const float *mu, *sigma;
-  float *partial;       // waves x kP
-  float *loss;          // waves
+  float *partial;       // parts x kP
+  float *loss;          // parts (kWide: every row's error, for loss_kernel)
 };
 
-__global__ __launch_bounds__(256) void train_rows_kernel(TrainArgs a) {
+// Gradient and squared error of a step's rows, a row per wave at a time (lane
+// = hidden unit, 224 multiply-adds and as many broadcasts). A part is what one
+// wave sums (kWide false: a training step of some thousand rows, four waves a
+// workgroup) or one workgroup of 12 waves (kWide: the one-off gradient over
+// many rows). What bounds the latter is the vector unit: 100,003 rows of 480
+// instructions are some 80 us on 256 CUs at full issue; with 64
+// workgroups of four waves it was 1.55 ms on 6 % of the chip. The workgroup's
+// sums meet in four LDS buffers, wave w in buffer w % 4 in order of w, so that
+// there are no more parts to write and add up than with 256 single waves, and
+// the result does not depend on timing.
+constexpr uint32_t kWideWaves = 12, kWideBufs = 4, kWideRows = 256;
+template <bool kWide>
+__global__ __launch_bounds__(kWide ? kWideWaves * kWave : 256) void train_rows_kernel(TrainArgs a) {
+  __shared__ float sAcc[kWide ? kWideBufs * kP : 1];
   __shared__ float sW1[kF * kH];
   __shared__ float sW2[kH * (kH + 1)];
   __shared__ float sB1[kH], sB2[kH], sW3[kH];
@@ -156,7 +169,7 @@ __global__ __launch_bounds__(256) void train_rows_kernel(TrainArgs a) {
   for (int i = 0; i < kH; ++i) gW2[i] = 0.f;
   float gb1 = 0.f, gb2 = 0.f, gw3 = 0.f, gb3 = 0.f, loss = 0.f;
   for (uint32_t r = wid; r < a.nrows; r += waves) {
-    const uint32_t row = a.idx[r];
+    const uint32_t row = a.idx ? a.idx[r] : r;
     const float xk = L < kF ? (a.x[(uint64_t)row * kF + L] - mu) * isg : 0.f;
     float h1 = b1;
 #pragma unroll
@@ -168,7 +181,11 @@ __global__ __launch_bounds__(256) void train_rows_kernel(TrainArgs a) {
     h2 = fmaxf(h2, 0.f);
     const float yhat = wave_sum_f32(h2 * w3) + b3;
     const float err = yhat - a.y[row];
-    loss += err * err;
+    if constexpr (kWide) {
+      if (L == 0) a.loss[r] = err;
+    } else {
+      loss += err * err;
+    }
     const float dy = 2.f * err * a.inv_batch;
     const float dh2 = h2 > 0.f ? dy * w3 : 0.f;
     float dh1 = 0.f;
@@ -184,6 +201,27 @@ __global__ __launch_bounds__(256) void train_rows_kernel(TrainArgs a) {
 #pragma unroll
     for (int k = 0; k < kF; ++k) gW1[k] += rdlane_f(xk, k) * dh1;
   }
+  if constexpr (kWide) {
+    const uint32_t w = threadIdx.x / kWave;
+    float *buf = sAcc + (w % kWideBufs) * kP;
+    for (uint32_t turn = 0; turn < kWideWaves / kWideBufs; ++turn) {
+      if (w / kWideBufs == turn) {
+        auto put = [&](int i, float v) { buf[i] = turn ? buf[i] + v : v; };
+#pragma unroll
+        for (int k = 0; k < kF; ++k) put(kOffW1 + k * kH + L, gW1[k]);
+        put(kOffB1 + L, gb1);
+#pragma unroll
+        for (int i = 0; i < kH; ++i) put(kOffW2 + i * kH + L, gW2[i]);
+        put(kOffB2 + L, gb2);
+        put(kOffW3 + L, gw3);
+        if (L == 0) put(kOffB3, gb3);
+      }
+      __syncthreads();
+    }
+    for (uint32_t i = threadIdx.x; i < (uint32_t)kP; i += blockDim.x)
+      a.partial[(uint64_t)blockIdx.x * kP + i] = (sAcc[i] + sAcc[kP + i]) + (sAcc[2 * kP + i] + sAcc[3 * kP + i]);
+    return;
+  }
   float *out = a.partial + (uint64_t)wid * kP;
 #pragma unroll
   for (int k = 0; k < kF; ++k) out[kOffW1 + k * kH + L] = gW1[k];
@@ -198,13 +236,42 @@ __global__ __launch_bounds__(256) void train_rows_kernel(TrainArgs a) {
   }
 }
 
-// grad[p] = sum over waves of partial[w][p], in wave order (deterministic).
-__global__ void reduce_partials_kernel(const float *__restrict__ partial, uint32_t waves, float *__restrict__ grad) {
+// loss[w] = the squared errors of rows w, w + parts, ... of a wide launch,
+// added one by one: the sums that `parts` single waves would make.
+__global__ void loss_kernel(const float *__restrict__ err, uint32_t rows, uint32_t parts, float *__restrict__ loss) {
+  const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
+  if (w >= parts) return;
+  float s = 0.f;
+  uint64_t r = w;
+  for (; r + 15ull * parts < rows; r += 16ull * parts) {
+    float e[16];
+#pragma unroll
+    for (uint32_t i = 0; i < 16; ++i) e[i] = err[r + (uint64_t)i * parts];
+#pragma unroll
+    for (uint32_t i = 0; i < 16; ++i) s += e[i] * e[i];
+  }
+  for (; r < rows; r += parts) s += err[r] * err[r];
+  loss[w] = s;
+}
+
+// grad[p] = sum over the parts of partial[w][p], in their order
+// (deterministic). Sixteen loads are in flight at a time: one after the other,
+// 256 parts were 58 us. The one-off gradient adds them up in 64 bits.
+template <typename Sum>
+__global__ void reduce_partials_kernel(const float *__restrict__ partial, uint32_t parts, float *__restrict__ grad) {
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= (uint32_t)kP) return;
-  float s = 0.f;
-  for (uint32_t w = 0; w < waves; ++w) s += partial[(uint64_t)w * kP + p];
-  grad[p] = s;
+  Sum s = 0;
+  uint32_t w = 0;
+  for (; w + 16 <= parts; w += 16) {
+    float v[16];
+#pragma unroll
+    for (uint32_t i = 0; i < 16; ++i) v[i] = partial[(uint64_t)(w + i) * kP + p];
+#pragma unroll
+    for (uint32_t i = 0; i < 16; ++i) s += v[i];
+  }
+  for (; w < parts; ++w) s += partial[(uint64_t)w * kP + p];
+  grad[p] = (float)s;
 }
 
 __global__ void adam_kernel(float *__restrict__ params, const float *__restrict__ grad, float *__restrict__ m,
@@ -500,28 +567,35 @@ int mce_mlp_grad(const mce_mlp *m, const float *x, const float *y, uint64_t rows
   if (rc) return rc;
   DevBuf b;
   float *dx, *dy, *dp, *dpart, *dloss, *dg;
-  uint32_t *didx;
-  const uint32_t blocks = (uint32_t)std::min<uint64_t>(64, (rows + 255) / 256 + 1), waves = blocks * 4;
+  // one workgroup of 12 waves a CU from 256 rows on (whole call, narrow and
+  // wide: 128 rows 0.25 and 0.25 ms, 256 0.31 and 0.25, 4,096 0.43 and 0.24,
+  // 100,003 2.06 and 0.57, 400,000 7.4 and 1.6)
+  const bool wide = rows >= kWideRows;
+  const uint32_t narrow = (uint32_t)std::min<uint64_t>(64, (rows + 255) / 256 + 1), sums = narrow * 4;
+  const uint32_t parts = wide ? 256 : sums;
   if ((rc = b.alloc((void **)&dx, sizeof(float) * rows * kF)) || (rc = b.alloc((void **)&dy, sizeof(float) * rows)) ||
-      (rc = b.alloc((void **)&dp, sizeof(float) * (kP + 2 * kF))) || (rc = b.alloc((void **)&didx, 4 * rows)) ||
-      (rc = b.alloc((void **)&dpart, sizeof(float) * kP * waves)) || (rc = b.alloc((void **)&dloss, 4 * waves)) ||
+      (rc = b.alloc((void **)&dp, sizeof(float) * (kP + 2 * kF))) ||
+      (rc = b.alloc((void **)&dpart, sizeof(float) * kP * parts)) || (rc = b.alloc((void **)&dloss, 4 * ((wide ? rows : 0) + sums))) ||
       (rc = b.alloc((void **)&dg, sizeof(float) * kP)))
     return rc;
-  std::vector<uint32_t> idx(rows);
-  std::iota(idx.begin(), idx.end(), 0u);
   MCE_HIP(hipMemcpy(dx, x, sizeof(float) * rows * kF, hipMemcpyHostToDevice));
   MCE_HIP(hipMemcpy(dy, y, sizeof(float) * rows, hipMemcpyHostToDevice));
-  MCE_HIP(hipMemcpy(didx, idx.data(), 4 * rows, hipMemcpyHostToDevice));
   MCE_HIP(hipMemcpy(dp, m->params, sizeof(float) * kP, hipMemcpyHostToDevice));
   MCE_HIP(hipMemcpy(dp + kP, m->mu, sizeof(float) * kF, hipMemcpyHostToDevice));
   MCE_HIP(hipMemcpy(dp + kP + kF, m->sigma, sizeof(float) * kF, hipMemcpyHostToDevice));
-  TrainArgs a{dx, dy, didx, (uint32_t)rows, 1.f / (float)rows, dp, dp + kP, dp + kP + kF, dpart, dloss};
-  train_rows_kernel<<<blocks, 256>>>(a);
-  reduce_partials_kernel<<<(kP + 255) / 256, 256>>>(dpart, waves, dg);
+  float *dsums = dloss + (wide ? rows : 0);
+  TrainArgs a{dx, dy, nullptr, (uint32_t)rows, 1.f / (float)rows, dp, dp + kP, dp + kP + kF, dpart, dloss};
+  if (wide) {
+    train_rows_kernel<true><<<parts, kWideWaves * kWave>>>(a);
+    loss_kernel<<<(sums + 63) / 64, 64>>>(dloss, (uint32_t)rows, sums, dsums);
+  } else {
+    train_rows_kernel<false><<<narrow, 256>>>(a);
+  }
+  reduce_partials_kernel<double><<<(kP + 255) / 256, 256>>>(dpart, parts, dg);
   MCE_HIP(hipGetLastError());
   MCE_HIP(hipMemcpy(grad, dg, sizeof(float) * kP, hipMemcpyDeviceToHost));
-  std::vector<float> hl(waves);
-  MCE_HIP(hipMemcpy(hl.data(), dloss, 4 * waves, hipMemcpyDeviceToHost));
+  std::vector<float> hl(sums);
+  MCE_HIP(hipMemcpy(hl.data(), dsums, 4 * sums, hipMemcpyDeviceToHost));
   if (loss_out) {
     double l = 0;
     for (float v : hl) l += v;
@@ -571,8 +645,8 @@ int mce_mlp_train(mce_mlp *m, const float *x, const float *y, uint64_t rows, con
     for (uint64_t s0 = 0; s0 < rows; s0 += batch) {
       const uint32_t nb = (uint32_t)std::min<uint64_t>(batch, rows - s0);
       TrainArgs a{dx, dy, didx + s0, nb, 1.f / (float)nb, dp, dp + kP, dp + kP + kF, dpart, dloss};
-      train_rows_kernel<<<blocks, 256>>>(a);
-      reduce_partials_kernel<<<(kP + 255) / 256, 256>>>(dpart, waves, dg);
+      train_rows_kernel<false><<<blocks, 256>>>(a);
+      reduce_partials_kernel<float><<<(kP + 255) / 256, 256>>>(dpart, waves, dg);
       ++step;
       const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
       adam_kernel<<<(kP + 255) / 256, 256>>>(dp, dg, dm, dv, o->lr, b1, b2, eps, o->weight_decay, c1, c2);
