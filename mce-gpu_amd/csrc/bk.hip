@@ -318,6 +318,7 @@ __device__ __forceinline__ void copy64(uint64_t *dst, const uint64_t *src, uint6
 // (which waits on both the LDS and the vector-memory counters).
 typedef __attribute__((address_space(3))) uint64_t lds_u64;
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
+typedef __attribute__((address_space(1))) unsigned long long glb_ull;
 typedef __attribute__((address_space(1))) uint64_t glb_u64;
 typedef __attribute__((address_space(1))) uint32_t glb_u32;
 
@@ -330,6 +331,11 @@ template <bool kL>
 __device__ __forceinline__ uint32_t ld32(const uint32_t *p, uint64_t i) {
   if constexpr (kL) return ((const lds_u32 *)p)[i];
   else return ((const glb_u32 *)p)[i];
+}
+template <bool kL>
+__device__ __forceinline__ void or64(uint64_t *p, uint64_t i, uint64_t v) {
+  if constexpr (kL) __hip_atomic_fetch_or((lds_ull *)p + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  else __hip_atomic_fetch_or((glb_ull *)p + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <bool kL>
 __device__ __forceinline__ void st64(uint64_t *p, uint64_t i, uint64_t v) {
@@ -1208,6 +1214,93 @@ __device__ __forceinline__ void clear_cover(uint64_t *cover) {
   __builtin_amdgcn_s_waitcnt(0);
 }
 
+// ---- out-lists against a subproblem's members ------------------------------
+// Which arcs of some vertices' out-lists lead into S (p members, ascending).
+// A step takes four arcs a lane; its chain is one load of arcs and one search
+// of log2 p steps, both for all four at once. (A list after the other with an
+// arc a lane waited for its offsets, its arcs and a search of its own: 2.6 us
+// a list, which was 50 to 90 % of the enumeration of graphs with up to some
+// 100 members a subproblem.) Enumeration in ms before and after: G(50,000, deg
+// 90) 3.26 -> 1.74, 100 block-model graphs of 500..900 3.16 -> 1.84, 301 of
+// 400..500 2.74 -> 1.72, 64 of 64..2,000 15.7 -> 11.6, 64 of 200..4,096 309 ->
+// 297, R-MAT 12 arcs 3.1 -> 2.35, R-MAT 14 21.0 -> 18.5.
+enum : int { kInGlb = 0, kInLds = 1, kAnywhere = 2 };
+template <int kS>
+__device__ __forceinline__ uint32_t ld_s(const uint32_t *p, uint32_t i) {
+  if constexpr (kS == kAnywhere) return p[i];
+  else return ld32<kS == kInLds>(p, i);
+}
+constexpr uint32_t kArcs = 4;
+// Places in S of the heads of list[k], list[k + step], ... (below n_arcs), or
+// kNone.
+template <int kS>
+__device__ __forceinline__ void find_arcs(const uint32_t *S, uint32_t p, const uint32_t *list, uint32_t k, uint32_t step,
+                                          uint32_t n_arcs, uint32_t (&j)[kArcs]) {
+  uint32_t y[kArcs];
+#pragma unroll
+  for (uint32_t m = 0; m < kArcs; ++m) {
+    y[m] = k + step * m < n_arcs ? list[k + step * m] : kNone;
+    j[m] = 0;
+  }
+  for (uint32_t st = 1u << (31 - __builtin_clz(p)); st; st >>= 1) {
+#pragma unroll
+    for (uint32_t m = 0; m < kArcs; ++m) {
+      const uint32_t t = j[m] + st;
+      const uint32_t v = ld_s<kS>(S, min(t, p) - 1u);
+      j[m] = t <= p && v < y[m] ? t : j[m];
+    }
+  }
+#pragma unroll
+  for (uint32_t m = 0; m < kArcs; ++m) {
+    const uint32_t v = ld_s<kS>(S, min(j[m], p - 1u));
+    j[m] = y[m] != kNone && v == y[m] ? j[m] : kNone;
+  }
+}
+// All arcs of n <= 64 lists (lane r < n: list [b, b + len)): hit gets a list's
+// number and the places of four of its arcs, lane by lane. Lists no longer
+// than they are many go a lane each, four arcs at a time (as many steps as
+// the longest has fours; a step of 16 lanes a list would leave most of them
+// idle: R-MAT 12 (ef 8) 0.54 -> 0.36 ms), lists of more than kLongList arcs one by one on the whole wave (one
+// on 16 lanes would keep the other three groups waiting; R-MAT 14 in ms: from
+// 64 arcs on 22.0, 128 19.8, 256 19.5, never 20.9), all others four at a time
+// on 16 lanes.
+constexpr uint32_t kLongList = 256;
+template <int kS, typename Hit>
+__device__ __forceinline__ void walk_lists(const uint32_t *oc, const uint32_t *S, uint32_t p, uint32_t n, uint64_t b,
+                                           uint32_t len, Hit hit) {
+  const uint32_t L = lane_id();
+  if (L >= n) len = 0;
+  const uint32_t most = wave_max(len);
+  uint32_t j[kArcs];
+  if (most <= n) {
+    for (uint32_t k0 = 0; k0 < most; k0 += kArcs) {
+      find_arcs<kS>(S, p, oc + b, k0, 1, len, j);
+      hit(L, j);
+    }
+    return;
+  }
+  const uint32_t gl = L & 15u, g = L >> 4, shorts = len <= kLongList ? len : 0u;
+  for (uint32_t r0 = 0; r0 < n; r0 += 4) {
+    const uint32_t r = r0 + g, at = 4 * (r & 63u);
+    const uint32_t bl = (uint32_t)__builtin_amdgcn_ds_bpermute((int)at, (int)(uint32_t)b);
+    const uint32_t bh = (uint32_t)__builtin_amdgcn_ds_bpermute((int)at, (int)(uint32_t)(b >> 32));
+    const uint32_t nr = (uint32_t)__builtin_amdgcn_ds_bpermute((int)at, (int)shorts), lr = r < n ? nr : 0u;
+    const uint32_t *list = oc + ((uint64_t)bh << 32 | bl);
+    for (uint32_t k0 = 0; ballot(k0 < lr) != 0; k0 += 16 * kArcs) {
+      find_arcs<kS>(S, p, list, k0 + gl, 16, lr, j);
+      hit(r, j);
+    }
+  }
+  for (uint64_t m = ballot(len > kLongList); m; m &= m - 1) {
+    const uint32_t r = ctz64(m), lr = rdlane(len, r);
+    const uint32_t *list = oc + rdlane64(b, r);
+    for (uint32_t k0 = 0; k0 < lr; k0 += kWave * kArcs) {
+      find_arcs<kS>(S, p, list, k0 + L, kWave, lr, j);
+      hit(r, j);
+    }
+  }
+}
+
 // Number of rows keep_chunk keeps from the q vertices in ids, for any q.
 __device__ __noinline__ __attribute__((not_tail_called)) uint32_t live_count_fn(ConstParams *kargs, const uint32_t *S,
                                                                                 uint32_t p, const uint32_t *ids, uint32_t q,
@@ -1221,6 +1314,7 @@ __device__ __noinline__ __attribute__((not_tail_called)) uint32_t live_count_fn(
   return n;
 }
 
+template <int kS>
 __device__ __noinline__ __attribute__((not_tail_called)) uint64_t live_rows_fn(ConstParams *kargs, const uint32_t *S,
                                                                                uint32_t p, const uint32_t *ids, uint32_t q) {
   const BkParams &pr = *(const BkParams *)(ConstParams *)uniform64((uint64_t)kargs);
@@ -1229,18 +1323,23 @@ __device__ __noinline__ __attribute__((not_tail_called)) uint64_t live_rows_fn(C
   const uint32_t L = lane_id();
   uint64_t keep = 0;
   for (uint32_t b = 0, k = 0; b < q; b += kWave, ++k) {
-    const uint32_t i = b + L;
-    bool any = false;
-    if (i < q) {
-      const uint32_t x = ids[i];
-      for (uint64_t t = pr.split[x], e = pr.rp[x + 1]; t < e && !any; ++t) {
-        const uint32_t y = pr.oc[t];
-        const uint32_t j = lower_bound_u32(S, p, y);
-        any = j < p && S[j] == y;
-      }
+    const uint32_t n = min(q - b, (uint32_t)kWave);
+    uint64_t t0 = 0;
+    uint32_t len = 0;
+    if (L < n) {
+      const uint32_t x = ids[b + L];
+      t0 = pr.split[x];
+      len = (uint32_t)(pr.rp[x + 1] - t0);
     }
-    const uint64_t m = ballot(any);
-    if (L == k) keep = m;
+    // a lane a list: most have a hit among their first arcs
+    bool any = false;
+    for (uint32_t k0 = 0; ballot(!any && k0 < len) != 0; k0 += kArcs) {
+      uint32_t j[kArcs];
+      find_arcs<kS>(S, p, pr.oc + t0, k0, 1, any ? 0u : len, j);
+      any = any || (j[0] & j[1] & j[2] & j[3]) != kNone;
+    }
+    const uint64_t mask = ballot(any);
+    if (L == k) keep = mask;
   }
   return keep;
 }
@@ -1249,9 +1348,10 @@ __device__ __forceinline__ uint32_t live_count(const uint32_t *S, uint32_t p, co
                                                uint64_t *cover) {
   return uniform(live_count_fn((ConstParams *)__builtin_amdgcn_kernarg_segment_ptr(), S, p, ids, q, cover));
 }
+template <int kS>
 __device__ __forceinline__ uint64_t live_rows(const uint32_t *S, uint32_t p, const uint32_t *ids, uint32_t q,
                                               uint32_t &nkeep) {
-  const uint64_t keep = live_rows_fn((ConstParams *)__builtin_amdgcn_kernarg_segment_ptr(), S, p, ids, q);
+  const uint64_t keep = live_rows_fn<kS>((ConstParams *)__builtin_amdgcn_kernarg_segment_ptr(), S, p, ids, q);
   nkeep = wave_sum(popc64(keep));
   return keep;
 }
@@ -1306,52 +1406,67 @@ __device__ __forceinline__ T lds_get(const __attribute__((address_space(3))) T *
 // filter: q0 may exceed 64 x 64 and the kept rows are found chunk by chunk
 // (keep_chunk) instead of from keep; their count, s.q, was taken by
 // live_count.
-__device__ __forceinline__ uint64_t build_bits(const BkParams &pr, Sub &s, const uint32_t *ids, uint32_t q0,
+template <bool kLA, bool kLX>
+__device__ __forceinline__ uint64_t build_bits(const BkParams &pr, const Sub &s, const uint32_t *ids, uint32_t q0,
                                                uint64_t keep, bool filter) {
   const uint32_t L = lane_id(), p = s.p, W = s.W, q = s.q;
   zero_words(s.A, (uint64_t)p * W);
   zero_words(s.XR, (uint64_t)q * W);
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  for (uint32_t i = 0; i < p; ++i) {
-    const uint32_t u = s.S[i];
-    const uint64_t b = pr.split[u], e = pr.rp[u + 1];
-    for (uint64_t k0 = b; k0 < e; k0 += kWave) {
-      const uint64_t k = k0 + L;
-      if (k < e) {
-        const uint32_t y = pr.oc[k];
-        const uint32_t j = lower_bound_u32(s.S, p, y);
-        if (j < p && s.S[j] == y) {
-          atomicOr((unsigned long long *)&s.A[(uint64_t)i * W + (j >> 6)], 1ull << (j & 63));
-          atomicOr((unsigned long long *)&s.A[(uint64_t)j * W + (i >> 6)], 1ull << (i & 63));
-        }
-      }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  for (uint32_t i0 = 0; i0 < p; i0 += kWave) {
+    const uint32_t n = min(p - i0, (uint32_t)kWave);
+    uint64_t b = 0;
+    uint32_t len = 0;
+    if (L < n) {
+      const uint32_t u = ld32<kLA>(s.S, i0 + L);
+      b = pr.split[u];
+      len = (uint32_t)(pr.rp[u + 1] - b);
     }
+    walk_lists<kLA ? kInLds : kInGlb>(pr.oc, s.S, p, n, b, len, [&](uint32_t r, const uint32_t (&j)[kArcs]) {
+      const uint32_t i = i0 + r;
+#pragma unroll
+      for (uint32_t m = 0; m < kArcs; ++m)
+        if (j[m] != kNone) {
+          or64<kLA>(s.A, (uint64_t)i * W + (j[m] >> 6), 1ull << (j[m] & 63));
+          or64<kLA>(s.A, (uint64_t)j[m] * W + (i >> 6), 1ull << (i & 63));
+        }
+    });
   }
   uint32_t base = 0;
   if (filter) clear_cover(s.cover);
   for (uint32_t b = 0, k = 0; b < q0; b += kWave, ++k) {
     const uint64_t km = filter ? keep_chunk(pr, s.S, p, ids, q0, b, s.cover) : rdlane64(keep, k);
-    if ((km >> L) & 1ull) {
-      const uint32_t x = ids[b + L];
-      uint64_t *row = s.XR + (uint64_t)(base + mbcnt(km)) * W;
-      for (uint64_t t = pr.split[x]; t < pr.rp[x + 1]; ++t) {
-        const uint32_t y = pr.oc[t];
-        const uint32_t j = lower_bound_u32(s.S, p, y);
-        if (j < p && s.S[j] == y) row[j >> 6] |= 1ull << (j & 63);
-      }
+    const uint32_t n = popc64(km);
+    if (n == 0) continue;
+    // the kept vertices, in order, to lanes 0.. (the others behind them)
+    const uint32_t x0 = b + L < q0 ? ids[b + L] : 0u;
+    const uint32_t dst = lane_in(km) ? mbcnt(km) : n + (L - mbcnt(km));
+    const uint32_t x = (uint32_t)__builtin_amdgcn_ds_permute((int)(dst * 4), (int)x0);
+    uint64_t t0 = 0;
+    uint32_t len = 0;
+    if (L < n) {
+      t0 = pr.split[x];
+      len = (uint32_t)(pr.rp[x + 1] - t0);
     }
-    base += popc64(km);
+    walk_lists<kLA ? kInLds : kInGlb>(pr.oc, s.S, p, n, t0, len, [&](uint32_t r, const uint32_t (&j)[kArcs]) {
+#pragma unroll
+      for (uint32_t m = 0; m < kArcs; ++m)
+        if (j[m] != kNone) or64<kLX>(s.XR, (uint64_t)(base + r) * W + (j[m] >> 6), 1ull << (j[m] & 63));
+    });
+    base += n;
   }
   fill_hash_terms(s);
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
   return full_word(q);
 }
 
-__device__ __noinline__ __attribute__((not_tail_called)) uint64_t build_bits_fn(ConstParams *kargs, uint32_t io, const uint32_t *ids, uint32_t q0,
-                                               uint64_t keep, uint32_t filter) {
+template <bool kLA, bool kLX>
+__device__ __noinline__ __attribute__((not_tail_called)) uint64_t build_bits_fn(ConstParams *kargs, uint32_t io,
+                                                                                const uint32_t *ids, uint32_t q0,
+                                                                                uint64_t keep, uint32_t filter) {
   const BkParams &pr = *(const BkParams *)(ConstParams *)uniform64((uint64_t)kargs);
-  Sub s = lds_get(&handover(uniform(io))->s);
-  return build_bits(pr, s, (const uint32_t *)uniform64((uint64_t)ids), uniform(q0), keep, uniform(filter) != 0);
+  const Sub s = lds_get(&handover(uniform(io))->s);
+  return build_bits<kLA, kLX>(pr, s, (const uint32_t *)uniform64((uint64_t)ids), uniform(q0), keep, uniform(filter) != 0);
 }
 
 // Pivot over P|X (index order) then the outside rows in E (row order): the
@@ -2652,8 +2767,10 @@ __device__ __forceinline__ void finish_bits(const BkParams &pr, Sub &s, const ui
                                             Clock<kStat> &clk) {
   clk.to(kBdInduced);
   lds_put(&handover(wa.io)->s, s);
-  const uint64_t E0 =
-      build_bits_fn((ConstParams *)__builtin_amdgcn_kernarg_segment_ptr(), wa.io, ids, q0, keep, filter);
+  ConstParams *ka = (ConstParams *)__builtin_amdgcn_kernarg_segment_ptr();
+  const uint64_t E0 = s.where == 3   ? build_bits_fn<true, true>(ka, wa.io, ids, q0, keep, filter)
+                      : s.where == 1 ? build_bits_fn<true, false>(ka, wa.io, ids, q0, keep, filter)
+                                     : build_bits_fn<false, false>(ka, wa.io, ids, q0, keep, filter);
   solve_bits<kWL, kStat>(pr, s, full_word(s.p), 0, E0, hist_lds, wa, clk);
 }
 
@@ -2804,7 +2921,7 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
           if (!bits) qb = q;
         }
         const uint64_t keep = !bits || filter ? 0ull
-                              : q > 2 * p     ? live_rows(pr.oc + s0, p, pr.oc + b0, q, qb)
+                              : q > 2 * p     ? live_rows<kInGlb>(pr.oc + s0, p, pr.oc + b0, q, qb)
                                               : all_rows(q);
         const Region rg = bits ? pool_take_wait<kFn>(pl, bits_want(p, qb, W, lv), bits_want_inner(p, qb, W, lv),
                                                 bits_fs(W, (qb + 63) / 64) * min(p, lv),
@@ -2867,7 +2984,7 @@ __global__ __launch_bounds__(max_wpg_of(kWL) * kWave, waves_per_simd_of(kWL)) vo
         const uint32_t W = (p + 63) / 64;
         const bool bits = kIPX && q <= kMaxXRows;
         uint32_t qk = q;
-        const uint64_t keep = !bits ? 0ull : q > 2 * p ? live_rows(t.S, p, t.XL, q, qk) : all_rows(q);
+        const uint64_t keep = !bits ? 0ull : q > 2 * p ? live_rows<kAnywhere>(t.S, p, t.XL, q, qk) : all_rows(q);
         if (!(bits ? place_bits(s, p, qk, W, rg.ptr, rg.bytes, hbm, pr.hbm_bytes, pr.stack_lds)
                    : place(s, p, q, W, kIPX, rg.ptr, rg.bytes, hbm, pr.hbm_bytes, pr.stack_lds))) {
           pool_put<kFn>(pl, rg);
