@@ -33,3 +33,21 @@ def test_lists_of_all_lengths(mce, oracle, a, b, extra):
                 res = dg.count(level=level, induced=2, worklist=1, **opts)
                 for k in ("count", "hist", "hash", "tree_nodes"):
                     assert res[k] == ref[k], (k, opts)
+
+
+@pytest.mark.parametrize("a,b,extra", [(20, 90, 300), (257, 300, 400), (1030, 1040, 500)])
+def test_features_count_inner_edges(mce, a, b, extra):
+    # up to and past the members that a wave keeps in LDS (1,024)
+    u, v, n = bipartite(a, b, extra, 5)
+    g = mce.from_edges(u, v, n=n)
+    with mce.DeviceGraph(g) as dg:
+        dg.order()
+        F = dg.features()
+        _, split, oc = dg.download()
+    rp = g.row_ptr.astype(np.int64)
+    split = split.astype(np.int64)
+    deg = rp[1:] - split
+    for x in list(np.argsort(-deg)[:6]) + list(range(0, n, max(n // 20, 1))):
+        P = oc[split[x]:rp[x + 1]]
+        inner = sum(int(np.isin(oc[split[w]:rp[w + 1]], P).sum()) for w in P)
+        assert abs(F[x, 7] - np.log1p(inner)) <= 1e-5 * max(1.0, np.log1p(inner))
