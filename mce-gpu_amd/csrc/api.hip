@@ -11,6 +11,8 @@
 #include <algorithm>
 #include <cmath>
 #include <string>
+#include <map>
+#include <mutex>
 #include <vector>
 
 #include "engine.hpp"
@@ -52,6 +54,37 @@ __global__ void validate_kernel(uint32_t n, const uint64_t *__restrict__ rp, con
       if (bad) atomicOr(err, bad);
     }
   }
+}
+
+// Streams of destroyed graphs, for the next ones on the device: making and
+// destroying a stream is 120 us, a third of a call on a graph of some hundred
+// vertices. At most four wait here (more are destroyed); each is idle and
+// belongs to one graph from take to give. Never torn down, as static objects
+// may outlive the HIP runtime.
+struct IdleStreams {
+  std::mutex m;
+  std::vector<hipStream_t> idle;
+  hipStream_t take() {
+    std::lock_guard<std::mutex> lock(m);
+    if (idle.empty()) return nullptr;
+    hipStream_t s = idle.back();
+    idle.pop_back();
+    return s;
+  }
+  bool give(hipStream_t s) {
+    hipStreamCaptureStatus c;
+    if (hipStreamIsCapturing(s, &c) != hipSuccess || c != hipStreamCaptureStatusNone) return false;
+    std::lock_guard<std::mutex> lock(m);
+    if (idle.size() >= 4) return false;
+    idle.push_back(s);
+    return true;
+  }
+};
+IdleStreams &idle_streams(int device) {
+  static std::mutex m;
+  static auto *all = new std::map<int, IdleStreams>;
+  std::lock_guard<std::mutex> lock(m);
+  return (*all)[device];
 }
 
 void fill_order_fields(const mce_graph *h, mce_result *res) {
@@ -137,7 +170,8 @@ int mce_graph_create(const mce_csr *csr, int device, mce_graph **out) {
     mce_graph_destroy(h);
     return rc;
   };
-  if (hipStreamCreateWithFlags(&h->s, hipStreamNonBlocking) != hipSuccess)
+  h->s = idle_streams(device).take();
+  if (!h->s && hipStreamCreateWithFlags(&h->s, hipStreamNonBlocking) != hipSuccess)
     return fail(set_error(MCE_EDEVICE, "stream creation failed"));
   DevGraph &g = h->g;
   g.n = csr->n;
@@ -181,7 +215,7 @@ int mce_graph_create(const mce_csr *csr, int device, mce_graph **out) {
 void mce_graph_destroy(mce_graph *h) {
   if (!h) return;
   hipSetDevice(h->device);
-  if (h->s) hipStreamSynchronize(h->s);
+  const bool clean = h->s && hipStreamSynchronize(h->s) == hipSuccess;
   h->ws.release();
   hipFree(h->g.rp);
   hipFree(h->g.ci);
@@ -190,7 +224,7 @@ void mce_graph_destroy(mce_graph *h) {
   hipFree(h->g.prio);
   hipFree(h->g.dplus);
   hipFree(h->g.core);
-  if (h->s) hipStreamDestroy(h->s);
+  if (h->s && !(clean && idle_streams(h->device).give(h->s))) hipStreamDestroy(h->s);
   delete h;
 }
 
@@ -447,8 +481,8 @@ static int count_impl(mce_graph *h, const mce_opts *opts, mce_result *res, bool 
     cleanup();
     return rc;
   }
-  std::vector<uint64_t> hh(kHistLen);
-  MCE_HIP(hipMemcpy(hh.data(), hist, sizeof(uint64_t) * kHistLen, hipMemcpyDeviceToHost));
+  std::vector<uint64_t> hh(kHistLen);  // (no clique past the largest)
+  MCE_HIP(hipMemcpy(hh.data(), hist, sizeof(uint64_t) * (std::min(out.max_size, kHistLen - 1) + 1), hipMemcpyDeviceToHost));
   if (res->hist && res->hist_len) {
     const uint32_t k = std::min<uint32_t>(res->hist_len, kHistLen);
     memcpy(res->hist, hh.data(), sizeof(uint64_t) * k);

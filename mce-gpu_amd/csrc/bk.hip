@@ -106,6 +106,8 @@ enum TaskKind : uint32_t { kTaskList = 0, kTaskBits = 1 };
 // realtime ticks without any they report a termination failure and exit
 // (default 120 s; BkParams::watchdog_ticks overrides it). A busy wave beats
 // once per kBeatNodes tree nodes.
+// HBM arena a wave up to which arenas are sized by the degree maxima
+constexpr uint64_t kSmallNeed = 16 << 10;
 constexpr uint64_t kWatchdogTicks = 12000000000ull;
 constexpr uint64_t kBeatNodes = 1u << 16;
 
@@ -3371,7 +3373,7 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
   if ((rc = dmalloc((void **)&acc, sizeof(unsigned long long) * (kAccN + 3), kWsAcc))) return rc;
   ticket = (uint32_t *)(acc + kAccN + 2);
   unsigned long long *need = acc + kAccN;
-  MCE_HIP(hipMemsetAsync(acc, 0, sizeof(unsigned long long) * (kAccN + 2), s));
+  MCE_HIP(hipMemsetAsync(acc, 0, sizeof(unsigned long long) * (kAccN + 3), s));
   // hub row filter: 64 words per wave, for every wave a launch can hold (four
   // per SIMD), taken before the arenas size themselves to what is left
   uint64_t *cover = nullptr;
@@ -3383,10 +3385,16 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
   // pass.
   uint64_t cap = cfg.hbm_bytes ? cfg.hbm_bytes : 16ull << 20;
   if (sc) cap = std::min<uint64_t>(cap, (sc->left() / wpg) & ~255ull);
-  need_kernel<<<(uint32_t)std::min<uint64_t>(1024, (n_items + 255) / 256), 256, 0, s>>>(g.rp, g.split, d_items, n_items, (uint32_t)cfg.level, cfg.ipx, cap, need);
-  unsigned long long hneed[2];
-  MCE_HIP(hipMemcpyAsync(hneed, need, sizeof(hneed), hipMemcpyDeviceToHost, s));
-  MCE_HIP(hipStreamSynchronize(s));
+  // (with small maxima the need of an item that has them all stands for the
+  // largest: the kernel, the copy and the wait for it are 25 us)
+  unsigned long long hneed[2] = {item_need(info.max_out_degree, info.max_in_degree, cfg.level != 1, cfg.ipx), 0};
+  if (cfg.level == 3)
+    hneed[0] = std::max<unsigned long long>(hneed[0], item_need(info.max_out_degree, info.max_in_degree, false, cfg.ipx));
+  if (sc || info.max_in_degree > kMaxXRows || hneed[0] > kSmallNeed || hneed[0] > cap) {
+    need_kernel<<<(uint32_t)std::min<uint64_t>(1024, (n_items + 255) / 256), 256, 0, s>>>(g.rp, g.split, d_items, n_items, (uint32_t)cfg.level, cfg.ipx, cap, need);
+    MCE_HIP(hipMemcpyAsync(hneed, need, sizeof(hneed), hipMemcpyDeviceToHost, s));
+    MCE_HIP(hipStreamSynchronize(s));
+  }
   if (sc && hneed[1])
     return set_error(MCE_ELIMIT, "%llu subproblems need more than the %llu scratch bytes per wave left (largest: %llu)",
                      (unsigned long long)hneed[1], (unsigned long long)cap, (unsigned long long)hneed[0]);
@@ -3554,7 +3562,6 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
   }
   hipEvent_t e0 = ev.a, e1 = ev.b;
   const auto host_t0 = std::chrono::steady_clock::now();
-  MCE_HIP(hipMemsetAsync(ticket, 0, sizeof(uint32_t), s));
   if (cfg.capture) {
     // one persistent launch captured into a graph: counters reset by a kernel
     // (no memset nodes), then the worker-list set-up and the enumeration
@@ -3612,9 +3619,11 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
   // items that did not fit: rerun them with arenas sized for the largest.
   // The deferred count is always read: an item deferred beyond what
   // need_kernel predicted would otherwise be lost without an error.
-  unsigned long long novf = 0;
-  MCE_HIP(hipMemcpyAsync(&novf, &acc[kAccOverflow], sizeof(novf), hipMemcpyDeviceToHost, s));
+  if (e1) MCE_HIP(hipEventRecord(e1, s));
+  unsigned long long h[kAccN];
+  MCE_HIP(hipMemcpyAsync(h, acc, sizeof(h), hipMemcpyDeviceToHost, s));
   MCE_HIP(hipStreamSynchronize(s));
+  const unsigned long long novf = h[kAccOverflow];
   if (novf > hneed[1])
     return set_error(MCE_EINTERNAL, "%llu items did not fit their arena, %llu predicted", novf, hneed[1]);
   if (novf) {
@@ -3648,15 +3657,11 @@ int bk_run(const DevGraph &g, const OrderInfo &info, const void *d_items, uint64
     MCE_HIP(hipMemsetAsync(ticket, 0, sizeof(uint32_t), s));
     if ((rc = dispatch(cfg.ipx, false, ls_max ? kStatLane : kStatNone, false, nullptr, p2, g2, wpg, lds, s)))
       return rc;
-    unsigned long long again = 0;
-    MCE_HIP(hipMemcpyAsync(&again, &acc[kAccOverflow], sizeof(again), hipMemcpyDeviceToHost, s));
+    if (e1) MCE_HIP(hipEventRecord(e1, s));
+    MCE_HIP(hipMemcpyAsync(h, acc, sizeof(h), hipMemcpyDeviceToHost, s));
     MCE_HIP(hipStreamSynchronize(s));
-    if (again != novf) return set_error(MCE_EINTERNAL, "items did not fit the large arena");
+    if (h[kAccOverflow] != novf) return set_error(MCE_EINTERNAL, "items did not fit the large arena");
   }
-  if (e1) MCE_HIP(hipEventRecord(e1, s));
-  unsigned long long h[kAccN];
-  MCE_HIP(hipMemcpyAsync(h, acc, sizeof(h), hipMemcpyDeviceToHost, s));
-  MCE_HIP(hipStreamSynchronize(s));
   float ms = 0;
   if (e0) {
     MCE_HIP(hipEventElapsedTime(&ms, e0, e1));

@@ -811,15 +811,15 @@ int peel(const DevGraph &g, hipStream_t s, OrderInfo *info) {
   const uint32_t row = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(g.m / n, 1), 1u << 20);
   // frontiers, and for a large graph degrees, alive lists and tail numbering
   uint32_t *buf = nullptr;
-  PeelState *hst = nullptr;
+  // (plain host memory: pinning and unpinning it is 65 us, its few copies are
+  // 100 bytes)
+  PeelState hst0{}, *hst = &hst0;
   int rc = MCE_OK;
   auto cleanup = [&]() {
     hipFree(buf);
-    if (hst) hipHostFree(hst);
   };
   const uint64_t words = (small ? 2ull * n : 6ull * n + 2 * kTailMax + kTailArcs / 2) + (sizeof(PeelState) + 15) / 16 * 4;
-  if (hipMalloc(&buf, sizeof(uint32_t) * words) != hipSuccess ||
-      hipHostMalloc(&hst, sizeof(PeelState), hipHostMallocDefault) != hipSuccess) {
+  if (hipMalloc(&buf, sizeof(uint32_t) * words) != hipSuccess) {
     cleanup();
     return set_error(MCE_ENOMEM, "peel: device allocation failed (n=%u)", n);
   }
