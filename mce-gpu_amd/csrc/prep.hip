@@ -62,13 +62,18 @@ struct PeelBufs {
 constexpr uint32_t kBlock = 256;
 constexpr uint32_t kPeelBlock = 1024;
 // One workgroup takes the whole peel of a graph of at most kTailMax vertices
-// and kTailArcs arcs, and the rest of a larger graph's peel once the alive
+// and kTailArcsEarly arcs, and the rest of a larger graph's peel once the alive
 // vertices and the arcs between them are as few: its round costs 2 to 3 us
 // against 6 us for a launch of the grid, but one CU takes only about 0.4 arcs
 // a nanosecond (measured on Chung-Lu 2^18: 3.3 ms against 10.8 ms a tail of
 // 32,768 vertices with no bound on its arcs).
 constexpr uint32_t kTailMax = 32768;
-constexpr uint32_t kTailArcs = 1u << 20;  // 2 MiB of 16-bit indices
+// Arcs of a tail (16-bit indices, 4 MiB), and those of a tail or a whole graph
+// before kTailRounds rounds: a peel that took many rounds has many small ones
+// left, which launches cost more than the one CU's 0.4 arcs a nanosecond (2^20
+// and 2^21 arcs in ms: R-MAT 18 6.4 and 5.1, Chung-Lu 2^18 5.7 and 5.0), one
+// that took few goes in large rounds (G(20,000, 600,000) 0.76 and 0.93).
+constexpr uint32_t kTailArcs = 1u << 21, kTailArcsEarly = 1u << 20, kTailRounds = 64;
 // With at most this many vertices, row offsets share the LDS with degrees.
 constexpr uint32_t kTailRowsMax = 16384;
 // A larger graph's rounds run on one workgroup while they hold about this
@@ -315,7 +320,7 @@ struct Rounds {
   }
 };
 
-// The whole peel of a graph of at most kTailMax vertices and kTailArcs arcs
+// The whole peel of a graph of at most kTailMax vertices and kTailArcsEarly arcs
 // (kAt kWholeRows: at most kTailRowsMax vertices).
 template <int kAt>
 __global__ __launch_bounds__(kPeelBlock) void kc_small(PeelBufs b) {
@@ -339,7 +344,8 @@ __global__ __launch_bounds__(kPeelBlock) void kc_small(PeelBufs b) {
 // (launches before that, and after the tail, do nothing): numbers the alive
 // vertices, then lays the arcs between them out as 16-bit indices.
 __device__ __forceinline__ bool tail_due(const PeelState *st) {
-  return st->mode == kModeLevel && st->acnt <= kTailMax && st->arcs <= kTailArcs;
+  return st->mode == kModeLevel && st->acnt <= kTailMax &&
+         st->arcs <= (st->round < kTailRounds ? kTailArcsEarly : kTailArcs);
 }
 __global__ __launch_bounds__(kBlock) void kc_number(PeelBufs b) {
   if (!tail_due(b.st)) return;
@@ -807,7 +813,7 @@ int peel(const DevGraph &g, hipStream_t s, OrderInfo *info) {
     return MCE_OK;
   }
   PeelBufs b{};
-  const bool small = n <= kTailMax && g.m <= kTailArcs;
+  const bool small = n <= kTailMax && g.m <= kTailArcsEarly;
   const uint32_t row = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(g.m / n, 1), 1u << 20);
   // frontiers, and for a large graph degrees, alive lists and tail numbering
   uint32_t *buf = nullptr;
